@@ -196,8 +196,8 @@ int qmr_supported_bf16_quantization(uint32_t bits, size_t group);
  *     The reference caps blocks at four RHS (src/gpu.rs:1136-1140). Buffers
  *     w, s, b, x, y; params rows, cols, bits, group, batch with
  *     1 <= batch <= 256; x [batch][cols], y [batch][rows] token-major;
- *     threads = rows*32. Q4/g64 runs on MFMA; meant for chunked prefill.
- *     Batches of up to eight run as successive blocks of up to four.
+ *     threads = rows*32. Five RHS or more run on MFMA in one pass, fewer as
+ *     a block; meant for chunked prefill.
  *   "matmul_affine_add" / "_bf16" / "_f16meta"
  *     y = r + W x, the down projection with the decoder's residual add
  *     (src/engine.rs:764-765). Buffers w, s, b, x, r, y; params as the
@@ -256,6 +256,13 @@ int qmr_supported_bf16_quantization(uint32_t bits, size_t group);
  *            products run on that kernel by default wherever it supports
  *            the view (16-byte aligned weights, cols % 32 == 0); rr = -1
  *            sends them to the vector-ALU kernels.
+ *   rr = -6: wide blocks on the wide kernel with ks = nw*100000 + ns*1000 +
+ *            ct*100 + rt (waves per workgroup, K splits, tiles of 16 RHS and
+ *            of 16 rows per workgroup; zero fields and ks = 0 leave them to
+ *            its planner). Wide blocks of more than four RHS run on that
+ *            kernel by default; any other rr runs them as blocks of four,
+ *            but for Q4, group 64, F32 or BF16 metadata, whole 256 columns
+ *            and more than eight RHS.
  * Shapes a forced kernel does not support fall back to the next one; pairs
  * that are not compiled fall back to the planner. */
 int qmr_set_gemv_plan(qmr_device *device, int rr, int ks);

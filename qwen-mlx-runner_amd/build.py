@@ -42,9 +42,7 @@ SOURCES = [
     ("affine_tile.hip", ["-x", "hip"]),
     ("dense_mfma.hip", ["-x", "hip"]),
     ("misc_kernels.hip", ["-x", "hip"]),
-    # MFMA accumulators in VGPRs: the wide kernel's FP32 epilogue adds into
-    # the same registers its bias MFMAs accumulate into.
-    ("wide_mfma.hip", ["-x", "hip", "-mllvm", "-amdgpu-mfma-vgpr-form"]),
+    ("wide_mfma.hip", ["-x", "hip"]),
 ]
 
 

@@ -224,13 +224,22 @@ size_t affine_tile_workspace(const TilePlan &pl, const AffineArgs &a);
 hipError_t launch_affine_tile(const AffineArgs &a, const TilePlan &pl, unsigned long long *partial,
                               uint32_t *counters, uint32_t epoch, const TileWait &wait, hipStream_t stream);
 
-// Wide block on MFMA (Q4/g64, F32 or BF16 metadata, batch up to 256): a prep
-// launch converts x into per-group images in `workspace` (wide_mfma_workspace
-// bytes), then the contraction launch. See wide_mfma.hip.
+// Wide block on MFMA (Q4/Q8, group 32/64/128, any metadata, batch up to 256):
+// a prep launch converts x into images in `workspace` (wide_mfma_workspace
+// bytes), the contraction, and with K splits the sum of their planes. See
+// wide_mfma.hip.
+struct WidePlan {
+    uint32_t rt = 0;   // 16-row tiles per workgroup; 0 = no plan
+    uint32_t ct = 0;   // 16-RHS tiles per workgroup
+    uint32_t nw = 0;   // waves (K classes) per workgroup, 4 or 8
+    uint32_t ns = 0;   // K splits across workgroups
+    uint32_t ups = 0;  // 128-column units per split (a multiple of nw)
+};
 bool wide_mfma_supported(const AffineArgs &a);
-size_t wide_mfma_workspace(const AffineArgs &a);
-hipError_t launch_wide_mfma(const AffineArgs &a, unsigned char *workspace, const DeviceLimits &lim,
-                            hipStream_t stream);
+// Non-zero fields of `force` (tuning hook) are kept.
+WidePlan plan_wide(const AffineArgs &a, const DeviceLimits &lim, const WidePlan &force = WidePlan{});
+size_t wide_mfma_workspace(const AffineArgs &a, const WidePlan &pl);
+hipError_t launch_wide_mfma(const AffineArgs &a, const WidePlan &pl, unsigned char *workspace, hipStream_t stream);
 // Host-side walk of every code, x-fragment and group-sum load the wide
 // contraction kernel issues for a shape with nrt row tiles per block: the
 // largest end (offset + size) of the in-range loads in the code view and in

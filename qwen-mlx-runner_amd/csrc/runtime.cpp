@@ -1309,11 +1309,35 @@ static int encode_command(qmr_command *command, const char *cname, qmr_buffer *c
             a.batch = qmr::starts_with(name, "matmul_") ? params[4] : 1;
             a.meta = meta;
             const bool fast_group = a.group == 32 || a.group == 64 || a.group == 128;
-            // The wide kernel takes RHS in blocks of 32 and measures about
-            // 33 us at 17408x5120 for any batch up to 32, against 15.8 us for
-            // one split-K block of four: batches of up to eight run as blocks.
-            if (wide && qmr::wide_mfma_supported(a) && a.batch > 8) {
-                const size_t need = qmr::wide_mfma_workspace(a);
+            // Wide blocks of five RHS on run on the wide kernel: against
+            // blocks of four, eight RHS take 20 us instead of 29 at
+            // 17408x5120, 8.0 instead of 8.5 at 1024x1024 (Q4). A forced plan
+            // is the block kernels' (rr == -6: this one's), and a static
+            // encode whose images don't fit its scratch runs as blocks; the
+            // large blocks of the usual format are refused there instead.
+            qmr::WidePlan wpl;
+            if (wide && a.batch > 4 && qmr::wide_mfma_supported(a)) {
+                const qmr::GemvPlan f = dev->forced_plan;
+                const uintptr_t al = reinterpret_cast<uintptr_t>(a.w) | reinterpret_cast<uintptr_t>(a.s) |
+                                     reinterpret_cast<uintptr_t>(a.b);
+                const bool large = a.batch > 8 && a.bits == 4 && a.group == 64 && a.meta != qmr::Meta::F16 &&
+                                   a.cols % 256 == 0 && al % 16 == 0;
+                if (large || f.rr == 0 || f.rr == -6) {
+                    qmr::WidePlan force;
+                    if (f.rr == -6) {
+                        const uint32_t ks = uint32_t(f.ks);
+                        force.rt = ks % 100;
+                        force.ct = ks / 100 % 10;
+                        force.ns = ks / 1000 % 100;
+                        force.nw = ks / 100000 % 10;
+                    }
+                    wpl = qmr::plan_wide(a, dev->limits, force);
+                    if (wpl.rt == 0) wpl = qmr::plan_wide(a, dev->limits);  // the pair is not compiled
+                    if (fixed && !large && qmr::wide_mfma_workspace(a, wpl) > QMR_STATIC_SCRATCH_BYTES) wpl = {};
+                }
+            }
+            if (wpl.rt > 0) {
+                const size_t need = qmr::wide_mfma_workspace(a, wpl);
                 unsigned char *images = fixed;
                 if (fixed) {
                     check_static_scratch(need, "wide-block activation images");
@@ -1330,10 +1354,10 @@ static int encode_command(qmr_command *command, const char *cname, qmr_buffer *c
                 if (!fixed) images = dev->ws_wide;
                 dev->last_hip = "wide_mfma_kernel";
                 start_gpu(dev);
-                e = qmr::launch_wide_mfma(a, images, dev->limits, dev->stream);
+                e = qmr::launch_wide_mfma(a, wpl, images, dev->stream);
             } else if (wide) {
-                // Wide blocks of up to eight RHS, and those outside the wide
-                // kernel's format, run as successive blocks of up to four RHS.
+                // Up to four RHS and what the wide kernel doesn't take:
+                // successive blocks of up to four RHS.
                 for (uint32_t t0 = 0; t0 < a.batch && e == hipSuccess; t0 += 4) {
                     qmr::AffineArgs sub = a;
                     sub.batch = a.batch - t0 < 4 ? a.batch - t0 : 4;

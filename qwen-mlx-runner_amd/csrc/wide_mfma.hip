@@ -1,43 +1,44 @@
-// Wide block (chunked prefill) on the matrix cores: Q4/g64 weights times up
-// to 256 RHS, y[t][r] = sum_c (q[r,c]*s[r,g] + b[r,g]) * x[t][c], computed
-// in the factored form
+// Wide block (chunked prefill) on the matrix cores: packed-affine weights
+// times up to 256 RHS, y[t][r] = sum_c (q[r,c]*s[r,g] + b[r,g]) * x[t][c],
+// computed in the factored form
 //     y[t][r] = sum_g ( s[r,g] * D[r,t,g] + b[r,g] * S[t,g] ),
 //     D[r,t,g] = sum_{c in g} q[r,c] * x[t,c],  S[t,g] = sum_{c in g} x[t,c].
-// D runs on v_mfma_f32_16x16x32_f16 with exact integer codes (f16
-// subnormals q*2^-20, as in mfma_common.hpp) against x split into hi/lo f16
-// parts, so it is accurate to about 2^-22; the scales multiply D in FP32 and
-// the bias term is an FP32 matrix product of S and b (v_mfma_f32_16x16x4_f32
-// over four groups at a time).
+// D runs on v_mfma_f32_16x16x32_f16 with exact integer codes (f16 subnormals,
+// as in mfma_common.hpp, or centred ones) against x split into hi/lo f16 parts, so it is
+// accurate to about 2^-22; the scales multiply D in FP32 and the bias term is
+// an FP32 matrix product of S and b (v_mfma_f32_16x16x4_f32 over four groups
+// at a time).
 //
-// Two launches:
-//   1. wide_prep_kernel turns x into one image per (quant group, block of 32
-//      RHS): the group's eight MFMA A fragments (2 K steps x 2 RHS tiles x
-//      hi/lo, 1 KB each, in lane order), the group sums S of the 32 RHS and
-//      the factor 2^(20+e) of the block's power-of-two scale 2^-e.
-//   2. wide_mfma_kernel: a workgroup of four waves (one per SIMD) owns
-//      16*NRT rows x 32 RHS. Wave w takes every fourth quant group, g = w
-//      (mod 4), so the four waves read the four 32-byte pieces of the same
-//      128-byte code lines at about the same time (one L2 fetch, three L1
-//      hits) and each x fragment is loaded once. A wave covers all row tiles
-//      and both RHS tiles (8 FP32 accumulators per lane and row tile; a
-//      second wave per SIMD gains nothing here, the vector ALU and the
-//      matrix cores of a SIMD barely overlap). Per group it loads the 8 x
-//      fragments (one group ahead) and one 8-byte code piece per row tile
-//      (the next group's piece is requested as soon as this one is unpacked)
-//      straight into registers. Scales (already multiplied by the image
-//      factors) and biases stream through LDS in chunks of 16 groups, two
-//      buffers, loaded by the whole workgroup one chunk ahead. At the end the
-//      four group classes meet in LDS and are added in a fixed order.
-// With NRT = 17 the 17408-row MLP matrix is 64 row blocks, which with four
-// 32-RHS blocks at 128 RHS is one workgroup per CU of the 256.
+// Launches: wide_prep_kernel (x images), wide_mfma_kernel and, where K is
+// split across workgroups, wide_sum_kernel.
+//
+// wide_mfma_kernel: a workgroup of NW waves owns 16*NRT rows x 16*NCT RHS
+// over one K split; wave w takes every NW-th 128-column unit (class w), all of
+// the workgroup's rows and RHS: 4*NRT*NCT FP32 accumulators per lane. Each
+// x fragment (1 KB) is loaded once per NRT tiles and each unpacked code is
+// used for NCT RHS tiles. Codes and x go straight to registers one unit ahead;
+// four consecutive lanes load 64 contiguous bytes of a code row, and the wave
+// turns a tile into operand order through its own piece of LDS (loading in
+// operand order, 16 rows for every 16 lanes, made the L1 look up 64 lines for
+// each 512 bytes). Metadata streams through LDS, expanded to FP32, a chunk of
+// four groups per class at a time. At the end the classes meet in LDS and are
+// added in a fixed order.
+//
+// What bounds it: up to 16 RHS the codes (17408x5120, Q4, 5 RHS: 21 us with the
+// prep launch, 50 MB; one wave in flight per SIMD and a prep of 5 us keep it
+// from the 11 us of a copy), then the matrix cores, which spend two products on
+// every code (hi, lo), together with the unpacking: 24 RHS 28 us, 64 RHS 48 us,
+// 128 RHS 75 us, 0.61 PFLOP/s of products. Streaming every operand through LDS
+// and staging it by the whole workgroup took 34, 62 and 73 us; blocks of four,
+// which Q8 and the other groups ran as, 165 us for 64 RHS over a Q8 5120x5120
+// (24 now).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cstdint>
-#include <mutex>
 #include <type_traits>
-#include <vector>
 
+#include "../../include/qmr.h"
 #include "kernels.hpp"
 #include "mfma_common.hpp"
 
@@ -47,63 +48,89 @@ namespace {
 using namespace mfma;
 
 typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u3 __attribute__((ext_vector_type(3)));
+typedef int i4 __attribute__((ext_vector_type(4)));
 
-constexpr int kPrepThreads = 256;
-constexpr int kKRanges = 4;                      // group classes (g mod 4) per workgroup
-constexpr int kWaves = kKRanges;                  // one wave per group class
-constexpr int kThreads = 64 * kWaves;
-constexpr int kRhsBlock = 32;                     // RHS per workgroup and per image
-constexpr int kFragBytes = 1024;                  // one MFMA A fragment (64 lanes x 16 B)
-constexpr int kImgS = 8 * kFragBytes;             // S[32] f32
-constexpr int kImgFac = kImgS + kRhsBlock * 4;    // factor f32
-constexpr int kImgBytes = 8448;                   // image stride (16-byte multiple)
-static_assert(kImgFac + 4 <= kImgBytes, "image layout");
-
-// Metadata chunk in LDS (one of two buffers): s' (f32) and b (f32 for F32
-// metadata, bf16 for BF16) of 16 groups, [row][group] with a pitch of 20
-// entries (4 mod 8: the 16 rows one read touches fall in 16 banks).
-constexpr int kCG = 16;  // groups per chunk: one quad per group class
-constexpr int kPitch = 20;
-template <int META>
-constexpr size_t meta_buf_bytes(int nrt) {
-    return size_t(16) * nrt * kPitch * (4 + (META == 0 ? 4 : 2));
+// Codes as f16: Q4 as subnormals (the code times 2^-20), Q8 as 1024 + code;
+// centred, less the middle of their range (8 or 128), which goes into the
+// group's bias as middle * scale. Uncentred, s * D and b * S are large and
+// cancel: at 5120 columns 2.4e-7 against 64 bits for Q4 and 2.6e-7 for Q8,
+// centred 1.4e-7 and 1.2e-7. (Q4 as 1024 + code: 1.3e-7, but 10% slower with
+// two RHS tiles; without the shifts, from subnormals of 2^-24, the matrix
+// cores' sums are off by 6e-6.)
+template <int BITS>
+constexpr int kWideExp = BITS == 4 ? 20 : 0;
+constexpr float middle_of(int bits) { return bits == 4 ? 8.f : 128.f; }
+template <int BITS, bool CENTRED>
+__device__ __forceinline__ h8 wide_unpack(const u2 &w) {
+    if constexpr (BITS == 4) {
+        const u4 c[1] = {u4{w.x, 0u, 0u, 0u}};
+        const h8 v = unpack<4>(c, 0);
+        return CENTRED ? v - __builtin_bit_cast(_Float16, uint16_t(0x0080)) : v;  // 8 * 2^-20
+    } else {
+        static_assert(CENTRED, "1024 + code");
+        const h8 v = __builtin_bit_cast(
+            h8, u4{(w.x & 0x00FF00FFu) | 0x64006400u, ((w.x >> 8) & 0x00FF00FFu) | 0x64006400u,
+                   (w.y & 0x00FF00FFu) | 0x64006400u, ((w.y >> 8) & 0x00FF00FFu) | 0x64006400u});
+        return v - _Float16(1152);
+    }
 }
-template <int META>
-constexpr size_t wide_lds_bytes(int nrt) {
-    const size_t meta = 2 * meta_buf_bytes<META>(nrt);
-    const size_t red = size_t(kKRanges) * nrt * 2 * 4 * 64 * 4;  // [class][rt][ct][v][lane] f32
-    return meta > red ? meta : red;
+
+constexpr int kPrepThreads = 1024;
+constexpr uint32_t kUnit = 128;                 // columns per unit: four K steps of the MFMA
+constexpr int kRhsBlock = 32;                   // RHS per image
+constexpr int kFragBytes = 1024;                // one MFMA A fragment (64 lanes x 16 B)
+constexpr int kImgS = 16 * kFragBytes;          // [quarter or half][32] f32 column sums
+constexpr int kImgBytes = 16896;                // image stride
+static_assert(kImgS + 4 * kRhsBlock * 4 <= kImgBytes, "image layout");
+
+// A wave's piece of LDS: codes on their way to operand order (64 bytes of each
+// row, one unit of Q4 or half a unit of Q8; rows 80 bytes apart so that
+// neither the writes nor the reads meet in a bank).
+constexpr int kCodePitch = 80;
+constexpr size_t code_bytes(int nrt) { return size_t(16) * nrt * kCodePitch; }
+// A chunk's metadata, two buffers: per row and class four scales, then the
+// same for the biases. The pitch puts the 16 rows of a read in 16 banks (and
+// with four waves and 8 row tiles it leaves room for two workgroups per CU).
+constexpr int meta_pitch(int nw) { return 4 * nw + 2; }
+constexpr size_t meta_bytes(int nrt, int nw) { return size_t(16) * nrt * meta_pitch(nw) * 8; }
+constexpr int kRedPad = 16;  // words between row tiles of the final planes
+constexpr size_t wide_lds_bytes(int nrt, int nct, int nw) {
+    const size_t red = size_t(nw > 4 ? 4 : nw) * nrt * (nct * 256 + kRedPad) * 4;  // [plane][rt][ct][v][lane] f32
+    return std::max(2 * meta_bytes(nrt, nw) + nw * code_bytes(nrt), red);
 }
 
 // Byte offsets of the contraction kernel's code, x-fragment and group-sum
 // loads, as the per-lane vector offset and the wave-uniform scalar offset of
-// a buffer load. A load outside its view (a row past the matrix, a group
-// past the row, an image past the last group) gets the vector offset kOut,
-// which by itself lies past every view's extent, so it reads zeros whether
-// or not the range check adds the scalar offset (kOut plus any scalar offset
-// here stays below 2^32); every other load has voffset + soffset + size
-// within its view. qmr_wide_address_extent walks every load the kernel can
-// issue through these functions on the host.
+// a buffer load. A load outside its view (a row past the matrix, columns past
+// the row, a unit past the split, an RHS tile past the images) gets the vector
+// offset kOut, which by itself lies past every view's extent, so it reads
+// zeros whether or not the range check adds the scalar offset (kOut plus any
+// scalar offset here stays below 2^32); every other load has voffset +
+// soffset + size within its view. qmr_wide_address_extent walks these on the
+// host.
 struct WideAddr {
-    uint32_t rows, G, ntb, row_bytes;
-    // The 8-byte code piece of lane (r16, q) in row tile rt of the row block
-    // at row0, quant group g (lanes q hold the group's four 16-column quarters).
-    __host__ __device__ uint32_t code_v(uint32_t row0, uint32_t rt, uint32_t r16, uint32_t q, uint32_t g) const {
-        return (row0 + 16 * rt + r16 < rows && g < G) ? (row0 + r16) * row_bytes + q * 8 : kOut;
+    uint32_t rows, units, ntb, row_bytes;
+    // Lane (row16, piece) loads 16 bytes of row row0 + 16 rt + row16 at byte
+    // 64 seg + 16 piece (a unit is one 64-byte segment of Q4, two of Q8).
+    __host__ __device__ uint32_t code_v(uint32_t row0, uint32_t rt, uint32_t row16, uint32_t piece, uint32_t seg) const {
+        return row0 + 16 * rt + row16 < rows && 64 * seg + 16 * piece < row_bytes ? (row0 + row16) * row_bytes + 16 * piece
+                                                                                 : kOut;
     }
-    __host__ __device__ uint32_t code_s(uint32_t rt, uint32_t g) const { return rt * 16 * row_bytes + g * 32; }
-    // Fragment f of group g's image for RHS block tb; lane l reads 16 bytes.
-    __host__ __device__ uint32_t frag_v(uint32_t lane, uint32_t g) const { return g < G ? lane * 16 : kOut; }
-    __host__ __device__ uint32_t frag_s(uint32_t g, uint32_t tb, uint32_t f) const {
-        return (g * ntb + tb) * uint32_t(kImgBytes) + f * uint32_t(kFragBytes);
+    __host__ __device__ uint32_t code_s(uint32_t rt, uint32_t seg) const { return rt * 16 * row_bytes + 64 * seg; }
+    // Fragment f = 2*ks + hl of RHS tile ct in unit u; lane l reads 16 bytes.
+    __host__ __device__ uint32_t frag_v(uint32_t lane, uint32_t u, uint32_t ct) const {
+        return u < units && ct < 2 * ntb ? lane * 16 : kOut;
     }
-    // Group sum of RHS 16 ct + r16 in block tb for group g0 + 4 q (lane
-    // (r16, q)); g0 = 16 c + class.
-    __host__ __device__ uint32_t sum_v(uint32_t g0, uint32_t q, uint32_t r16, uint32_t ct) const {
-        return g0 + 4 * q < G ? q * 4 * ntb * uint32_t(kImgBytes) + uint32_t(kImgS) + r16 * 4 + ct * 64 : kOut;
+    __host__ __device__ uint32_t frag_s(uint32_t u, uint32_t ct, uint32_t f) const {
+        return (u * ntb + (ct >> 1)) * uint32_t(kImgBytes) + ((ct & 1) * 8 + f) * uint32_t(kFragBytes);
     }
-    __host__ __device__ uint32_t sum_s(uint32_t g0, uint32_t tb) const {
-        return (g0 * ntb + tb) * uint32_t(kImgBytes);
+    // Sum of RHS 16 ct + r16 over quarter `sub` of unit u (group 32) or half
+    // `sub` (the other groups).
+    __host__ __device__ uint32_t sum_at(uint32_t u, uint32_t sub, uint32_t ct, uint32_t r16) const {
+        return u < units && ct < 2 * ntb
+                   ? (u * ntb + (ct >> 1)) * uint32_t(kImgBytes) + uint32_t(kImgS) + sub * (kRhsBlock * 4) + (ct & 1) * 64 + r16 * 4
+                   : kOut;
     }
 };
 
@@ -112,469 +139,678 @@ struct WideParams {
     const void *s;
     const void *b;
     const float *x;
-    float *y;
-    const unsigned char *img;  // [G][NTB] images of kImgBytes
-    uint32_t rows, cols, n;    // n = RHS count
-    uint32_t ntb;              // 32-RHS blocks
-    uint32_t nrb;              // row blocks
+    float *y;              // output, or the first K split's plane
+    unsigned char *img;    // [units][ntb] images of kImgBytes
+    int *expo;             // [ns * nw][32 ntb] exponents e of the images' 2^-e
+    uint32_t rows, cols, n;       // n = RHS count
+    uint32_t group;
+    uint32_t units, groups;       // 128-column units (the last may be partial) and quant groups per row
+    uint32_t ntb, ncb;            // 32-RHS images, RHS blocks of the contraction
+    uint32_t nrb, ns, ups;        // row blocks, K splits, units per split
+    uint32_t plane;               // floats between K splits' planes (0: one split)
     uint32_t w_bytes, m_bytes, img_bytes;  // extents of the views
 };
 
-// ---- 1. Activation images. grid (G, NTB), 256 threads: thread -> RHS
-// tid/8 of the block and the 8 columns 8*(tid%8).. of the group, which is
-// code word tid%8 of every row: K step tid%2, lane group tid/2 of the MFMA
-// fragments. ----
-__global__ __launch_bounds__(kPrepThreads) void wide_prep_kernel(WideParams p) {
-    __shared__ float red[kPrepThreads / 64];
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const uint32_t g = blockIdx.x, tb = blockIdx.y;
-    const uint32_t tt = uint32_t(tid) >> 3, c = uint32_t(tid) & 7;
-    const uint32_t t = tb * kRhsBlock + tt;
+// ---- 1. Activation images: one workgroup per (RHS tile, K class), every wave
+// one unit at a time, lane (t16, c4) the columns 8*c4.. of the four K steps of
+// RHS t16. The scale 2^-e is shared by an RHS's units of one class, so that
+// the contraction can accumulate over them. ----
+template <int BITS>
+__global__ __launch_bounds__(kPrepThreads) void wide_prep_kernel(WideParams p, uint32_t nw) {
+    constexpr uint32_t kWavesP = kPrepThreads / 64;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    __shared__ uint32_t red[kWavesP][16];
+    const uint32_t ct = blockIdx.x % (2 * p.ntb), cls = blockIdx.x / (2 * p.ntb);
+    const uint32_t split = cls / nw, w = cls % nw;
+    const uint32_t u0 = split * p.ups, u1 = min(u0 + p.ups, p.units);
+    const uint32_t t16 = uint32_t(lane) & 15, c4 = uint32_t(lane) >> 4;
+    const uint32_t t = ct * 16 + t16;
     const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float *>(p.x), 0, int(p.n * p.cols * 4u), kRsrcWord3);
-    float xv[8];
-    load_x8(xv, xr, t, g * 64 + 8 * c, p.cols, t < p.n);
-    float sum = 0.f, mx = 0.f;
+    const uint32_t first = u0 + w + uint32_t(wave) * nw, step = kWavesP * nw;
+    auto load = [&](float (&xv)[4][8], uint32_t u) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        sum += xv[j];
-        mx = fmaxf(mx, fabsf(xv[j]));
+        for (uint32_t ks = 0; ks < 4; ++ks)
+            load_x8(xv[ks], xr, t, u * kUnit + 32 * ks + 8 * c4, p.cols, t < p.n && u < u1);
+    };
+    uint32_t mb = 0;
+    auto largest = [&](const float (&xv)[4][8]) {
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) mb = max(mb, __float_as_uint(xv[ks][j]) & 0x7FFFFFFFu);
+    };
+    float x0[4][8];
+    load(x0, first);
+    largest(x0);
+    for (uint32_t u = first + step; u < u1; u += step) {
+        float xv[4][8];
+        load(xv, u);
+        largest(xv);
     }
-    group_reduce<8>(sum, mx);  // one RHS: 8 consecutive lanes
-    float m = mx;
-#pragma unroll
-    for (int o = 8; o < 64; o <<= 1) m = fmaxf(m, __shfl_xor(m, o));
-    if (lane == 0) red[tid >> 6] = m;
+    mb = max(mb, uint32_t(__shfl_xor(int(mb), 16)));
+    mb = max(mb, uint32_t(__shfl_xor(int(mb), 32)));
+    if (lane < 16) red[wave][lane] = mb;
     __syncthreads();
-    m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    const uint32_t mb = __float_as_uint(m);
+    mb = red[0][t16];
+#pragma unroll
+    for (uint32_t v = 1; v < kWavesP; ++v) mb = max(mb, red[v][t16]);
     int e = 0;
     if (mb != 0u && mb < 0x7F800000u) {
         e = int(mb >> 23) - 127 - 14;  // max * 2^-e in [2^14, 2^15) for normal max
         e = e < -100 ? -100 : (e > 100 ? 100 : e);
     }
     const float sc = __uint_as_float(uint32_t(127 - e) << 23);
-    unsigned char *img = const_cast<unsigned char *>(p.img) + (size_t(g) * p.ntb + tb) * kImgBytes;
-    const uint32_t ks = c & 1, q = c >> 1, ct = tt >> 4;
-    const uint32_t ln = q * 16 + (tt & 15);
-    uint32_t hw[4], lw[4];
+    if (tid < 16) p.expo[size_t(cls) * (kRhsBlock * p.ntb) + t] = e;
+    auto store = [&](const float (&xv)[4][8], uint32_t u) {
+        unsigned char *img = p.img + (size_t(u) * p.ntb + (ct >> 1)) * kImgBytes;
+        unsigned char *frag = img + (ct & 1) * 8 * kFragBytes + lane * 16;
+        float quarter[4];  // this lane's part of the sum of each K step's 32 columns
 #pragma unroll
-    for (int e2 = 0; e2 < 4; ++e2) {
-        const float v0 = xv[k_of<4>(2 * e2)] * sc;
-        const float v1 = xv[k_of<4>(2 * e2 + 1)] * sc;
-        const h2 hh = __builtin_convertvector(f2{v0, v1}, h2);
-        const h2 ll = __builtin_convertvector(f2{v0 - static_cast<float>(hh.x), v1 - static_cast<float>(hh.y)}, h2);
-        hw[e2] = __builtin_bit_cast(uint32_t, hh);
-        lw[e2] = __builtin_bit_cast(uint32_t, ll);
+        for (int ks = 0; ks < 4; ++ks) {
+            const float(&v)[8] = xv[ks];
+            quarter[ks] = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+            u4 hw, lw;
+#pragma unroll
+            for (int e2 = 0; e2 < 4; ++e2) {
+                const float v0 = v[k_of<BITS>(2 * e2)], v1 = v[k_of<BITS>(2 * e2 + 1)];
+                hw[e2] = hi_pair(v0, v1, sc);
+                lw[e2] = lo_pair(v0, v1, sc, hw[e2]);
+            }
+            *reinterpret_cast<u4 *>(frag + 2 * ks * kFragBytes) = hw;
+            *reinterpret_cast<u4 *>(frag + (2 * ks + 1) * kFragBytes) = lw;
+        }
+        // Sums of the unit's quarters (group 32) or halves, with the codes'
+        // power of two, so that b * S adds to s * D.
+        const float cs = sc * (1.f / float(1u << kWideExp<BITS>));
+        float *S = reinterpret_cast<float *>(img + kImgS) + (ct & 1) * 16 + t16;
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            quarter[ks] += __shfl_xor(quarter[ks], 16);
+            quarter[ks] += __shfl_xor(quarter[ks], 32);
+        }
+        if (c4 == 0) {
+            if (p.group == 32) {
+#pragma unroll
+                for (int ks = 0; ks < 4; ++ks) S[ks * kRhsBlock] = quarter[ks] * cs;
+            } else {
+                S[0] = (quarter[0] + quarter[1]) * cs;
+                S[kRhsBlock] = (quarter[2] + quarter[3]) * cs;
+            }
+        }
+    };
+    if (first < u1) store(x0, first);
+    for (uint32_t u = first + step; u < u1; u += step) {
+        float xv[4][8];
+        load(xv, u);
+        store(xv, u);
     }
-    unsigned char *frag = img + ((ks * 2 + ct) * 2) * kFragBytes + ln * 16;
-    *reinterpret_cast<u4 *>(frag) = u4{hw[0], hw[1], hw[2], hw[3]};
-    *reinterpret_cast<u4 *>(frag + kFragBytes) = u4{lw[0], lw[1], lw[2], lw[3]};
-    if (c == 0) reinterpret_cast<float *>(img + kImgS)[tt] = sum;
-    if (tid == 0) reinterpret_cast<float *>(img + kImgFac)[0] = __uint_as_float(uint32_t(127 + kCodeExp<4> + e) << 23);
 }
 
-// One Q4 word (8 codes) as a B operand, in k_of order.
-__device__ __forceinline__ h8 unpack_word(uint32_t wd) {
-    const u4 c[1] = {u4{wd, 0u, 0u, 0u}};
-    return unpack<4>(c, 0);
-}
-
-// ---- 2. The contraction. grid: row blocks (padded to a multiple of 8) x
-// NTB, 256 threads. Lane (r16, q): row r16 of every row tile, K chunk q of
-// every K step; D element v of a tile is RHS 4q + v of its 16-RHS tile. ----
-template <int META, int NRT>
-__global__ __launch_bounds__(kThreads, 1) void wide_mfma_kernel(WideParams p) {
+// ---- 2. The contraction. Lane (r16, q) of a wave: row r16 of every row
+// tile, K chunk q of every K step; D element v of a tile is RHS 4q + v. ----
+template <int BITS, int META, bool G32, bool CENTRED, int NRT, int NCT, int NW_>
+__global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
+    constexpr uint32_t NW = NW_;
     constexpr int ROWS = 16 * NRT;
-    constexpr int BSZ = META == 0 ? 4 : 2;
-    constexpr size_t BUF = meta_buf_bytes<META>(NRT);
+    constexpr int SEG = BITS / 4;         // 64-byte code segments per unit
+    constexpr int KPS = 4 / SEG;          // K steps per segment
+    constexpr int KG = G32 ? 1 : 2;       // K steps per group (or half of 128)
+    constexpr int SL = 4 / KG;            // slots (groups or halves of 128) per unit
+    constexpr uint32_t UPC = 4 / SL;      // units per chunk: four slots, one bias product
+    constexpr int THREADS = 64 * NW_, PITCH = meta_pitch(NW_);
+    constexpr int PER_T = (NRT + 7) / 8;  // metadata items per thread and chunk
+    constexpr int RJ = (ROWS + 63) / 64;  // waves' worth of rows
+    constexpr uint32_t BSZ = META == 0 ? 4 : 2;
     extern __shared__ __align__(16) unsigned char lds[];
     const int tid = threadIdx.x;
-    const int kr = __builtin_amdgcn_readfirstlane(tid >> 6);  // the wave's group class (uniform)
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);  // the wave's K class (uniform)
     const int lane = tid & 63;
     const int r16 = lane & 15, q = lane >> 4;
-    // XCD-aware order: workgroup i runs on XCD i % 8, so the NTB workgroups
-    // of one row block (which read the same codes at about the same time)
-    // share an XCD and its L2.
+    unsigned char *turn = lds + 2 * meta_bytes(NRT, NW_) + size_t(wv) * code_bytes(NRT);
+    // XCD-aware order: workgroup i runs on XCD i % 8, so the RHS blocks of one
+    // row block (which read the same codes at about the same time) share an
+    // XCD and its L2.
     const uint32_t xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
-    const uint32_t tb = slot % p.ntb;
-    const uint32_t rb = (slot / p.ntb) * 8 + xcd;
-    if (rb >= p.nrb) return;
-    const uint32_t row0 = rb * ROWS;
-    const uint32_t G = p.cols / 64;
-    const uint32_t nch = (G + kCG - 1) / kCG;
-    const uint32_t row_bytes = p.cols / 2;
-    const WideAddr A{p.rows, G, p.ntb, row_bytes};
+    const uint32_t cb = slot % p.ncb, pair = (slot / p.ncb) * 8 + xcd;
+    if (pair >= p.nrb * p.ns) return;
+    const uint32_t rb = pair % p.nrb, split = pair / p.nrb;
+    const uint32_t row0 = rb * ROWS, ct0 = cb * NCT;
+    const uint32_t u0 = split * p.ups, u1 = min(u0 + p.ups, p.units);
+    const WideAddr A{p.rows, u1, p.ntb, p.cols / (32 / BITS) * 4};
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint32_t *>(p.w), 0, int(p.w_bytes), kRsrcWord3);
-    const __amdgpu_buffer_rsrc_t ir = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<unsigned char *>(p.img), 0, int(p.img_bytes), kRsrcWord3);
+    const __amdgpu_buffer_rsrc_t ir = __builtin_amdgcn_make_buffer_rsrc(p.img, 0, int(p.img_bytes), kRsrcWord3);
     const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p.s), 0, int(p.m_bytes), kRsrcWord3);
     const __amdgpu_buffer_rsrc_t br = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p.b), 0, int(p.m_bytes), kRsrcWord3);
-    const uint32_t m_pitch = G * BSZ;
     const f4 zero{0.f, 0.f, 0.f, 0.f};
-    float *red = reinterpret_cast<float *>(lds);  // final reduction [class][row tile][ct][v][lane]
 
-    // Metadata chunk c (groups 16c..16c+15) of all the workgroup's rows,
-    // staged by every thread: item (row, j) = groups 16c+4j..16c+4j+3 of one
-    // row; thread tid always has j = tid % 4, so it needs the image factors
-    // of 4 groups only. Past the matrix (rows or groups) everything is zero.
-    constexpr int ITEMS = ROWS * 4;
-    constexpr int PER_T = (ITEMS + kThreads - 1) / kThreads;
-    using Raw = std::conditional_t<META == 0, u4, u2>;
+    // ---- codes: lane (row16, piece) loads 16 bytes of a row of every tile.
+    const uint32_t row16 = uint32_t(lane) >> 2, piece = uint32_t(lane) & 3;
+    const uint32_t code_base = (row0 + row16) * A.row_bytes + 16 * piece;
+    const uint32_t tiles_in = row0 + row16 < p.rows ? (p.rows - row0 - row16 + 15) / 16 : 0;  // tiles with a row in the matrix
+    u4 raw[SEG][NRT];
+    auto load_codes = [&](u4 (&dst)[NRT], uint32_t u, int sg) {
+        const uint32_t seg = u * SEG + uint32_t(sg);
+        const uint32_t tiles = u < u1 && 64 * seg + 16 * piece < A.row_bytes ? tiles_in : 0u;
+#pragma unroll
+        for (int rt = 0; rt < NRT; ++rt)
+            dst[rt] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                 wr, int(uint32_t(rt) < tiles ? code_base : kOut), int(A.code_s(uint32_t(rt), seg)), 0));
+    };
+    auto put_codes = [&](const u4 (&src)[NRT]) {
+#pragma unroll
+        for (int rt = 0; rt < NRT; ++rt)
+            *reinterpret_cast<u4 *>(turn + (rt * 16 + row16) * kCodePitch + piece * 16) = src[rt];
+    };
+    // ---- metadata of chunk c (units u0 + UPC*NW*c ..): item (row, j) = eight
+    // consecutive groups of one row. A window of whole words that holds them
+    // and lies inside the view is loaded; the groups are shifted into place
+    // when they are used.
+    const uint32_t gpu = kUnit / p.group;      // groups per unit
+    const uint32_t gpc = gpu * UPC * NW;       // groups per chunk: 4 NW (group 128: 2 NW)
+    const uint32_t ipr = gpc / 8;              // items per row
+    const uint32_t ish = 31u - __builtin_clz(ipr);
+    const uint32_t mj = uint32_t(tid) & (ipr - 1);
+    const uint32_t g_first = gpu * u0, g_end = min(p.groups, gpu * u1);
+    constexpr uint32_t WIN = META == 0 ? 8 : 5;  // words of a window
     struct MStage {
-        Raw s[PER_T], b[PER_T];
-        float fac[4];
+        u4 s0[PER_T], b0[PER_T];
+        std::conditional_t<META == 0, u4, uint32_t> s1[PER_T], b1[PER_T];
     };
-    const uint32_t mj = uint32_t(tid) & 3;
-    auto meta_issue = [&](MStage &st, uint32_t c) {
-        const uint32_t g4 = c * kCG + 4 * mj;  // first group of this thread's items
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const uint32_t g = g4 + uint32_t(k);
-            const uint32_t off = g < G ? (g * p.ntb + tb) * kImgBytes + kImgFac : kOut;
-            st.fac[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ir, int(off), 0, 0));
-        }
+    auto item_row = [&](int i) { return (uint32_t(tid) + uint32_t(i) * THREADS) >> ish; };
+    auto item_at = [&](uint32_t rl, uint32_t c) { return ((row0 + rl) * p.groups + g_first + c * gpc + 8 * mj) * BSZ; };
+    auto window = [&](uint32_t at) { return min(at & ~3u, p.m_bytes - 4 * WIN); };
+    auto item_live = [&](uint32_t rl, uint32_t c) {
+        return rl < uint32_t(ROWS) && row0 + rl < p.rows && g_first + c * gpc + 8 * mj < g_end;
+    };
+    auto load_meta = [&](MStage &st, uint32_t c) {
 #pragma unroll
         for (int i = 0; i < PER_T; ++i) {
-            const uint32_t it = uint32_t(tid) + uint32_t(i) * kThreads;
-            const uint32_t rl = it >> 2;
-            const bool live = it < uint32_t(ITEMS) && row0 + rl < p.rows && g4 < G;
-            const uint32_t moff = live ? (row0 + rl) * m_pitch + g4 * BSZ : kOut;
+            const uint32_t rl = item_row(i);
+            const uint32_t at = item_live(rl, c) ? window(item_at(rl, c)) : kOut;
+            st.s0[i] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(sr, int(at), 0, 0));
+            st.b0[i] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(br, int(at), 0, 0));
             if constexpr (META == 0) {
-                st.s[i] = __builtin_amdgcn_raw_buffer_load_b128(sr, int(moff), 0, 0);
-                st.b[i] = __builtin_amdgcn_raw_buffer_load_b128(br, int(moff), 0, 0);
+                st.s1[i] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(sr, int(at + 16u), 0, 0));
+                st.b1[i] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(br, int(at + 16u), 0, 0));
             } else {
-                st.s[i] = __builtin_bit_cast(u2, __builtin_amdgcn_raw_buffer_load_b64(sr, int(moff), 0, 0));
-                st.b[i] = __builtin_bit_cast(u2, __builtin_amdgcn_raw_buffer_load_b64(br, int(moff), 0, 0));
+                st.s1[i] = __builtin_amdgcn_raw_buffer_load_b32(sr, int(at + 16u), 0, 0);
+                st.b1[i] = __builtin_amdgcn_raw_buffer_load_b32(br, int(at + 16u), 0, 0);
             }
         }
     };
-    auto meta_commit = [&](const MStage &st, uint32_t c) {
-        unsigned char *buf = lds + (c & 1) * BUF;
-        float *ms = reinterpret_cast<float *>(buf);
-        unsigned char *mb = buf + size_t(ROWS) * kPitch * 4;
+    // The window's elements from `skip` on (0, or 1 for a row that starts
+    // inside a word; more only where the view ends, handled word by word).
+    auto eight = [&](float (&out)[8], const u4 &w0, const auto &w1, uint32_t skip) {
+        uint32_t w[WIN];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) w[k] = w0[k];
+        if constexpr (META == 0) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) w[4 + k] = w1[k];
+        } else {
+            w[4] = w1;
+        }
+        const uint32_t words = META == 0 ? skip : skip >> 1;  // at most WIN - 1: the item starts inside the view
+        for (uint32_t i = 0; i < WIN - 1 && i < words; ++i) {
+#pragma unroll
+            for (uint32_t k = 0; k + 1 < WIN; ++k) w[k] = w[k + 1];
+        }
+        if constexpr (META == 0) {
+#pragma unroll
+            for (int k = 0; k < 8; ++k) out[k] = __uint_as_float(w[k]);
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const uint32_t v = __builtin_amdgcn_alignbit(w[k + 1], w[k], (skip & 1) * 16);
+                out[2 * k] = meta_f32<META>(v & 0xFFFFu);
+                out[2 * k + 1] = META == 1 ? __uint_as_float(v & 0xFFFF0000u) : meta_f32<META>(v >> 16);
+            }
+        }
+    };
+    auto put_meta = [&](const MStage &st, uint32_t c) {
+        float *ms = reinterpret_cast<float *>(lds + (c & 1) * meta_bytes(NRT, NW_));
+        float *mb = ms + ROWS * PITCH;
 #pragma unroll
         for (int i = 0; i < PER_T; ++i) {
-            const uint32_t it = uint32_t(tid) + uint32_t(i) * kThreads;
-            const uint32_t rl = it >> 2;
-            if (it < uint32_t(ITEMS)) {
-                float sv[4];
-                if constexpr (META == 0) {
+            const uint32_t rl = item_row(i);
+            const uint32_t at = item_at(rl, c), skip = item_live(rl, c) ? (at - window(at)) / BSZ : 0u;
+            float sv[8], bv[8];
+            eight(sv, st.s0[i], st.s1[i], skip);
+            eight(bv, st.b0[i], st.b1[i], skip);
+            const uint32_t g = g_first + c * gpc + 8 * mj;
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) sv[k] = __uint_as_float(st.s[i][k]);
-                } else {
+            for (uint32_t k = 0; k < 8; ++k) {  // past the split's groups there may be a neighbour's
+                sv[k] = g + k < g_end ? sv[k] : 0.f;
+                bv[k] = g + k < g_end ? CENTRED ? __builtin_fmaf(middle_of(BITS), sv[k], bv[k]) : bv[k] : 0.f;
+            }
+            if (rl >= uint32_t(ROWS)) continue;
+            // Unit NW*i + class of the chunk: slots 4*class + 2*i + half
+            // (group 32: 4*class + quarter); a group of 128 fills both halves.
+            float *s_row = ms + rl * PITCH, *b_row = mb + rl * PITCH;
+            if constexpr (G32) {
 #pragma unroll
-                    for (int k = 0; k < 2; ++k) {
-                        sv[2 * k] = __uint_as_float(st.s[i][k] << 16);
-                        sv[2 * k + 1] = __uint_as_float(st.s[i][k] & 0xFFFF0000u);
-                    }
+                for (int k = 0; k < 8; k += 2) {
+                    *reinterpret_cast<f2 *>(s_row + 8 * mj + k) = f2{sv[k], sv[k + 1]};
+                    *reinterpret_cast<f2 *>(b_row + 8 * mj + k) = f2{bv[k], bv[k + 1]};
                 }
-                *reinterpret_cast<float4 *>(ms + rl * kPitch + 4 * mj) =
-                    float4{sv[0] * st.fac[0], sv[1] * st.fac[1], sv[2] * st.fac[2], sv[3] * st.fac[3]};
-                *reinterpret_cast<Raw *>(mb + (rl * kPitch + 4 * mj) * BSZ) = st.b[i];
+            } else if (p.group == 64) {
+                const uint32_t ul = 4 * mj, sl = (ul % NW) * 4 + (ul / NW) * 2;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    *reinterpret_cast<f2 *>(s_row + sl + 4 * k) = f2{sv[2 * k], sv[2 * k + 1]};
+                    *reinterpret_cast<f2 *>(b_row + sl + 4 * k) = f2{bv[2 * k], bv[2 * k + 1]};
+                }
+            } else {
+#pragma unroll
+                for (uint32_t k = 0; k < 8; ++k) {
+                    const uint32_t ul = 8 * mj + k, sl = (ul % NW) * 4 + (ul / NW) * 2;
+                    *reinterpret_cast<f2 *>(s_row + sl) = f2{sv[k], sv[k]};
+                    *reinterpret_cast<f2 *>(b_row + sl) = f2{bv[k], bv[k]};
+                }
             }
         }
     };
+    // ---- x
+    u4 xf[4][NCT][2];  // a unit's K steps; whole words: halves carried across the loop would be taken apart and put together
+    auto load_x = [&](u4 (&dst)[NCT][2], uint32_t u, uint32_t ks) {
+#pragma unroll
+        for (int ct = 0; ct < NCT; ++ct) {
+            const int v = int(A.frag_v(uint32_t(lane), u, ct0 + uint32_t(ct)));
+#pragma unroll
+            for (int hl = 0; hl < 2; ++hl)
+                dst[ct][hl] = __builtin_bit_cast(
+                    u4, __builtin_amdgcn_raw_buffer_load_b128(ir, v, int(A.frag_s(u, ct0 + uint32_t(ct), 2 * ks + uint32_t(hl))), 0));
+        }
+    };
+    // Bias A operands of chunk c: lane (t16, q) the sum of slot q.
+    auto load_s = [&](float (&sop)[NCT], uint32_t c) {
+        const uint32_t u = u0 + c * UPC * NW + uint32_t(wv) + (G32 ? 0u : NW * (uint32_t(q) >> 1));
+#pragma unroll
+        for (int ct = 0; ct < NCT; ++ct)
+            sop[ct] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                ir, int(A.sum_at(u, G32 ? uint32_t(q) : uint32_t(q) & 1, ct0 + uint32_t(ct), uint32_t(r16))), 0, 0));
+    };
 
-    // The wave's share: all row tiles, groups kr, kr+4, ...
+    f4 acc[NRT][NCT];
+    float sa[NCT];
     {
-        constexpr int NTW = NRT;
-        // Code piece of row tile rt: words 2q, 2q+1 of the group for row
-        // row0 + 16 rt + r16 (WideAddr: rows past the matrix and groups past
-        // the row read zeros through the vector offset).
-        u2 cw[NTW];
-        auto load_codes = [&](int rt, uint32_t g) {
-            cw[rt] = __builtin_bit_cast(
-                u2, __builtin_amdgcn_raw_buffer_load_b64(wr, int(A.code_v(row0, uint32_t(rt), uint32_t(r16), uint32_t(q), g)),
-                                                         int(A.code_s(uint32_t(rt), g)), 0));
-        };
-        // x fragments of group g: f = (ks*2 + ct)*2 + hl, lane i at 16 i
-        // (past the last group: zeros).
-        auto load_x = [&](h8 (&xf)[8], uint32_t g) {
-            const int xo = int(A.frag_v(uint32_t(lane), g));
+        const uint32_t u = u0 + uint32_t(wv);
+        MStage st;
+        load_meta(st, 0);
 #pragma unroll
-            for (int f = 0; f < 8; ++f)
-                xf[f] = __builtin_bit_cast(
-                    h8, __builtin_amdgcn_raw_buffer_load_b128(ir, xo, int(A.frag_s(g, tb, uint32_t(f))), 0));
-        };
-        // Bias A operands of chunk c: S[16c + 4q + kr][16 ct + r16].
-        auto load_s = [&](float (&sop)[2], uint32_t c) {
-            const uint32_t g0 = c * kCG + uint32_t(kr);
+        for (int sg = 0; sg < SEG; ++sg) load_codes(raw[sg], u, sg);
 #pragma unroll
-            for (int ct = 0; ct < 2; ++ct)
-                sop[ct] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                    ir, int(A.sum_v(g0, uint32_t(q), uint32_t(r16), uint32_t(ct))), int(A.sum_s(g0, tb)), 0));
-        };
+        for (int ks = 0; ks < 4; ++ks) load_x(xf[ks], u, uint32_t(ks));
+        load_s(sa, 0);
+        __builtin_amdgcn_sched_barrier(0);  // every request before any use
+        put_meta(st, 0);
+    }
+#pragma unroll
+    for (int rt = 0; rt < NRT; ++rt)
+#pragma unroll
+        for (int ct = 0; ct < NCT; ++ct) acc[rt][ct] = zero;
+    lds_barrier();
 
-        f4 acc[NTW][2];
-        // One group (chunk buffer cb, class step i): codes of g in cw (their
-        // successors, group g+4, requested as each piece is unpacked), x
-        // fragments of g in xf. Software-pipelined by row tile: step rt
-        // issues the 8 MFMAs of tile rt and, on the vector ALU, the epilogue
-        // of tile rt-1 and the unpacking of tile rt+1; a scheduling barrier
-        // keeps the steps apart, which bounds the live registers.
-        auto group = [&](const h8 (&xf)[8], uint32_t g, const float *ms, int i) {
-            const float *msw = ms + r16 * kPitch + 4 * i + kr;
-            h8 bc[2][2];  // [tile parity][K step]
-            f4 dp0 = zero, dp1 = zero;
-            float svp = 0.f;
-            bc[0][0] = unpack_word(cw[0].x);
-            bc[0][1] = unpack_word(cw[0].y);
-            load_codes(0, g + 4);
-            float svn = msw[0];
-            __builtin_amdgcn_sched_barrier(0);
+    // Codes of K step k of the segment in the turn buffer, row tile rt, as a B operand.
+    auto operand = [&](int rt, int k) {
+        const unsigned char *row = turn + (rt * 16 + r16) * kCodePitch;
+        if constexpr (BITS == 4) return u2{*reinterpret_cast<const uint32_t *>(row + 16 * k + 4 * q), 0u};
+        else return *reinterpret_cast<const u2 *>(row + 32 * k + 8 * q);
+    };
+    // The wave's units of the split, the last one perhaps past it (its loads
+    // read zeros): the loop body has no branch, so every wait counts on the
+    // loads really in flight.
+    const uint32_t nu = (u1 - u0 + NW - 1) / NW;
+    for (uint32_t c = 0;; ++c) {
+        const float *ms = reinterpret_cast<const float *>(lds + (c & 1) * meta_bytes(NRT, NW_)) + r16 * PITCH + 4 * wv;
+        const float *mb = ms + ROWS * PITCH;
+        MStage st;
+        float sb[NCT];
+        load_meta(st, c + 1);
+        load_s(sb, c + 1);
+        const uint32_t n = min(UPC, nu - c * UPC);
+        uint32_t h = 0;
+        do {
+            const uint32_t u = u0 + (c * UPC + h) * NW + uint32_t(wv), un = u + NW;
 #pragma unroll
-            for (int rt = 0; rt < NTW; ++rt) {
-                const h8 b0 = bc[rt & 1][0], b1 = bc[rt & 1][1];
-                f4 d0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[0], b0, zero, 0, 0, 0);
-                f4 d1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[2], b0, zero, 0, 0, 0);
-                d0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[1], b0, d0, 0, 0, 0);
-                d1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[3], b0, d1, 0, 0, 0);
-                d0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[4], b1, d0, 0, 0, 0);
-                d1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[6], b1, d1, 0, 0, 0);
-                d0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[5], b1, d0, 0, 0, 0);
-                d1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[7], b1, d1, 0, 0, 0);
-                if (rt > 0) {
+            for (int sg = 0; sg < SEG; ++sg) {
+                put_codes(raw[sg]);
+                load_codes(raw[sg], un, sg);
+                wave_lds_sync();
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        acc[rt - 1][0][v] = __builtin_fmaf(svp, dp0[v], acc[rt - 1][0][v]);
-                        acc[rt - 1][1][v] = __builtin_fmaf(svp, dp1[v], acc[rt - 1][1][v]);
+                for (int k0 = 0; k0 < KPS; k0 += KG) {
+                    const int ks = sg * KPS + k0, sl = ks / KG;  // the group's first K step, its slot
+                    // Software-pipelined by row tile: step rt issues tile rt's
+                    // products and, on the vector ALU, the epilogue of tile
+                    // rt-1 and the unpacking of tile rt+1; codes and scales
+                    // are read from LDS two tiles ahead.
+                    h8 op[2][KG];
+                    u2 w[2][KG];
+                    float sv[3];
+                    auto fetch = [&](int rt) {
+#pragma unroll
+                        for (int k = 0; k < KG; ++k) w[rt & 1][k] = operand(rt, k0 + k);
+                        sv[rt % 3] = ms[rt * 16 * PITCH + SL * h + sl];
+                    };
+                    auto open = [&](int rt) {
+#pragma unroll
+                        for (int k = 0; k < KG; ++k) op[rt & 1][k] = wide_unpack<BITS, CENTRED>(w[rt & 1][k]);
+                    };
+                    f4 d[2][NCT];
+                    auto close = [&](int rt) {
+#pragma unroll
+                        for (int ct = 0; ct < NCT; ++ct)
+#pragma unroll
+                            for (int v = 0; v < 4; ++v)
+                                acc[rt][ct][v] = __builtin_fmaf(sv[rt % 3], d[rt & 1][ct][v], acc[rt][ct][v]);
+                    };
+                    fetch(0);
+                    if (NRT > 1) fetch(1);
+                    open(0);
+#pragma unroll
+                    for (int rt = 0; rt < NRT; ++rt) {
+                        __builtin_amdgcn_sched_barrier(0);
+                        // All hi products before the lo ones: half the error
+                        // of hi and lo in turn (2.4e-7 against 4.4e-7 at 5120
+                        // columns, Q4), a quarter of lo first.
+#pragma unroll
+                        for (int hl = 0; hl < 2; ++hl)
+#pragma unroll
+                            for (int k = 0; k < KG; ++k)
+#pragma unroll
+                                for (int ct = 0; ct < NCT; ++ct)
+                                    d[rt & 1][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                                        __builtin_bit_cast(h8, xf[ks + k][ct][hl]), op[rt & 1][k],
+                                        k == 0 && hl == 0 ? zero : d[rt & 1][ct], 0, 0, 0);
+                        if (rt + 1 < NRT) open(rt + 1);
+                        if (rt > 0) close(rt - 1);
+                        if (rt + 2 < NRT) fetch(rt + 2);
                     }
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int k = 0; k < KG; ++k) load_x(xf[ks + k], un, uint32_t(ks + k));
+                    close(NRT - 1);
                 }
-                if (rt + 1 < NTW) {
-                    bc[(rt + 1) & 1][0] = unpack_word(cw[rt + 1].x);
-                    bc[(rt + 1) & 1][1] = unpack_word(cw[rt + 1].y);
-                    load_codes(rt + 1, g + 4);
+                wave_lds_sync();
+            }
+            // Bias of the chunk's four slots, acc += S x b, after its first
+            // unit: b * S cancels most of s * D, so in the middle the sums
+            // stray half as far.
+            if (h == 0) {
+#pragma unroll
+                for (int rt = 0; rt < NRT; ++rt) {
+                    const float bv = mb[rt * 16 * PITCH + q];
+#pragma unroll
+                    for (int ct = 0; ct < NCT; ++ct)
+                        acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(sa[ct], bv, acc[rt][ct], 0, 0, 0);
                 }
-                svp = svn;
-                if (rt + 1 < NTW) svn = msw[(rt + 1) * 16 * kPitch];
-                dp0 = d0;
-                dp1 = d1;
-                __builtin_amdgcn_sched_barrier(0);
             }
+        } while (++h < n);
+        if ((c + 1) * UPC >= nu) break;
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                acc[NTW - 1][0][v] = __builtin_fmaf(svp, dp0[v], acc[NTW - 1][0][v]);
-                acc[NTW - 1][1][v] = __builtin_fmaf(svp, dp1[v], acc[NTW - 1][1][v]);
-            }
-        };
-        // Bias of the wave's four groups of a chunk: acc += S x b.
-        auto bias = [&](const float (&sop)[2], const unsigned char *mb) {
-#pragma unroll
-            for (int rt = 0; rt < NTW; ++rt) {
-                const uint32_t e = (rt * 16 + r16) * kPitch + 4 * q + kr;
-                float bvv;
-                if constexpr (META == 0)
-                    bvv = reinterpret_cast<const float *>(mb)[e];
-                else
-                    bvv = __uint_as_float(uint32_t(reinterpret_cast<const uint16_t *>(mb)[e]) << 16);
-#pragma unroll
-                for (int ct = 0; ct < 2; ++ct)
-                    acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(sop[ct], bvv, acc[rt][ct], 0, 0, 0);
-            }
-        };
-
-        // All first requests in flight together (chunk 0's metadata, the
-        // first group's codes and x, chunk 0's S), then chunk 0 into LDS.
-        h8 xa[8], xb[8];
-        float sa[2], sb[2];
-        {
-            MStage st;
-            meta_issue(st, 0);
-            load_x(xa, uint32_t(kr));
-            load_s(sa, 0);
-#pragma unroll
-            for (int rt = 0; rt < NTW; ++rt) load_codes(rt, uint32_t(kr));
-            __builtin_amdgcn_sched_barrier(0);  // every request before any use
-            meta_commit(st, 0);
-        }
-#pragma unroll
-        for (int rt = 0; rt < NTW; ++rt) acc[rt][0] = acc[rt][1] = zero;
+        for (int ct = 0; ct < NCT; ++ct) sa[ct] = sb[ct];
+        put_meta(st, c + 1);
         lds_barrier();
-        // Chunk c: this wave's groups 16c + kr + 4i, i = 0..3. The next
-        // chunk's metadata is requested first and committed to the other
-        // buffer at the end (after the last chunk: zeros, never read), so the
-        // loop body has no branch.
-        for (uint32_t c = 0; c < nch; ++c) {
-            const unsigned char *buf = lds + (c & 1) * BUF;
-            const float *ms = reinterpret_cast<const float *>(buf);
-            const unsigned char *mb = buf + size_t(ROWS) * kPitch * 4;
-            const uint32_t g = c * kCG + uint32_t(kr);
-            MStage st;
-            meta_issue(st, c + 1);
-            load_s(sb, c + 1);
-            load_x(xb, g + 4);
-            group(xa, g, ms, 0);
-            load_x(xa, g + 8);
-            group(xb, g + 4, ms, 1);
-            load_x(xb, g + 12);
-            group(xa, g + 8, ms, 2);
-            load_x(xa, g + 16);
-            group(xb, g + 12, ms, 3);
-            bias(sa, mb);
-            sa[0] = sb[0];
-            sa[1] = sb[1];
-            meta_commit(st, c + 1);
-            lds_barrier();
-        }
+    }
 
-        // The group classes meet in LDS (the metadata buffers are free).
+    // ---- the classes meet in LDS, each wave's sums times 2^(e + code
+    // exponent), and are added in order. A wave stores 64 rows of an RHS at a
+    // time.
+    lds_barrier();  // every wave is done with its piece
+    float *red = reinterpret_cast<float *>(lds);
+    constexpr int TILE = NCT * 256 + kRedPad;
+    constexpr uint32_t PLANES = NW > 4 ? 4 : NW;
 #pragma unroll
-        for (int rt = 0; rt < NTW; ++rt)
+    for (int ct = 0; ct < NCT; ++ct) {
+        const uint32_t t = (ct0 + uint32_t(ct)) * 16 + uint32_t(q) * 4;
+        i4 e{0, 0, 0, 0};
+        if (ct0 + uint32_t(ct) < 2 * p.ntb)
+            e = *reinterpret_cast<const i4 *>(p.expo + size_t(split * NW + uint32_t(wv)) * (kRhsBlock * p.ntb) + t);
 #pragma unroll
-            for (int ct = 0; ct < 2; ++ct)
+        for (int rt = 0; rt < NRT; ++rt)
 #pragma unroll
-                for (int v = 0; v < 4; ++v)
-                    red[(((kr * NRT + rt) * 2 + ct) * 4 + v) * 64 + lane] = acc[rt][ct][v];
+            for (int v = 0; v < 4; ++v) acc[rt][ct][v] = ldexpf(acc[rt][ct][v], e[v] + kWideExp<BITS>);
+    }
+    auto place = [&](int rt, int ct, int v) -> float & {
+        return red[((wv % int(PLANES)) * NRT + rt) * TILE + (ct * 4 + v) * 64 + lane];
+    };
+    if (wv < int(PLANES)) {
+#pragma unroll
+        for (int rt = 0; rt < NRT; ++rt)
+#pragma unroll
+            for (int ct = 0; ct < NCT; ++ct)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) place(rt, ct, v) = acc[rt][ct][v];
     }
     lds_barrier();
-    // Wave w writes the (row tile, ct, v) combinations w, w+4, ...: lane
-    // (r16, q) holds row 16 rt + r16 and RHS 16 ct + 4 q + v; the four group
-    // classes are added in order.
-    for (int cmb = kr; cmb < NRT * 8; cmb += kWaves) {
-        float sum = 0.f;
+    if constexpr (NW > PLANES) {
+        if (wv >= int(PLANES)) {
 #pragma unroll
-        for (int k = 0; k < kKRanges; ++k) sum += red[(k * NRT * 8 + cmb) * 64 + lane];
-        const uint32_t rt = uint32_t(cmb) >> 3, ct = (uint32_t(cmb) >> 2) & 1, v = uint32_t(cmb) & 3;
-        const uint32_t r = row0 + rt * 16 + uint32_t(r16);
-        const uint32_t t = tb * kRhsBlock + ct * 16 + uint32_t(q) * 4 + v;
-        if (r < p.rows && t < p.n) p.y[size_t(t) * p.rows + r] = sum;
+            for (int rt = 0; rt < NRT; ++rt)
+#pragma unroll
+                for (int ct = 0; ct < NCT; ++ct)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) place(rt, ct, v) += acc[rt][ct][v];
+        }
+        lds_barrier();
+    }
+    float *out = p.y + size_t(split) * p.plane;
+    const uint32_t rows_here = min(uint32_t(ROWS), p.rows - row0);
+    for (uint32_t i = uint32_t(wv); i < uint32_t(RJ) * 16 * NCT; i += NW) {
+        const uint32_t tl = i / RJ, rl = (i % RJ) * 64 + uint32_t(lane);  // RHS 16 ct + 4 q + v of the block, row
+        const uint32_t t = ct0 * 16 + tl;
+        if (t >= p.n) break;  // uniform
+        if (rl < rows_here) {
+            const uint32_t at = (rl >> 4) * TILE + ((tl >> 4) * 4 + (tl & 3)) * 64 + ((tl >> 2) & 3) * 16 + (rl & 15);
+            float sum = 0.f;
+#pragma unroll
+            for (uint32_t k = 0; k < PLANES; ++k) sum += red[k * NRT * TILE + at];
+            out[size_t(t) * p.rows + row0 + rl] = sum;
+        }
     }
 }
 
-// Resident workgroups per CU of a kernel instance (as the runtime computes
-// it from registers and LDS); cached.
-uint32_t resident_per_cu(const void *kernel, size_t lds) {
-    struct Entry {
-        const void *k;
-        size_t lds;
-        uint32_t n;
-    };
-    static std::mutex mu;
-    static std::vector<Entry> cache;
-    std::lock_guard<std::mutex> lock(mu);
-    for (const Entry &e : cache)
-        if (e.k == kernel && e.lds == lds) return e.n;
-    int n = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, kThreads, lds) != hipSuccess || n < 1) n = 1;
-    cache.push_back(Entry{kernel, lds, uint32_t(n)});
-    return uint32_t(n);
+// ---- 3. The K splits' planes, added in split order. ----
+__global__ __launch_bounds__(256) void wide_sum_kernel(const float *__restrict__ planes, float *__restrict__ y,
+                                                       uint32_t count, uint32_t ns) {
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < count; i += gridDim.x * 256) {
+        float v = 0.f;
+        for (uint32_t k = 0; k < ns; ++k) v += planes[size_t(k) * count + i];
+        y[i] = v;
+    }
 }
 
-template <int META, int NRT>
-hipError_t launch_nrt(WideParams p, hipStream_t stream) {
-    auto kernel = wide_mfma_kernel<META, NRT>;
-    constexpr size_t lds = wide_lds_bytes<META>(NRT);
-    {
-        const hipError_t e = raise_lds_limit(reinterpret_cast<const void *>(kernel), lds);
-        if (e != hipSuccess) return e;
-    }
-    p.nrb = (p.rows + 16 * NRT - 1) / (16 * NRT);
-    const uint32_t grid = (p.nrb + 7) / 8 * 8 * p.ntb;  // XCD-aware order; surplus workgroups exit
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), lds, stream, p);
+template <int BITS, int META, bool G32, bool CENTRED, int NRT, int NCT, int NW>
+hipError_t launch_instance(const WideParams &p, hipStream_t stream) {
+    auto kernel = wide_mfma_kernel<BITS, META, G32, CENTRED, NRT, NCT, NW>;
+    constexpr size_t lds = wide_lds_bytes(NRT, NCT, NW);
+    const hipError_t e = raise_lds_limit(reinterpret_cast<const void *>(kernel), lds);
+    if (e != hipSuccess) return e;
+    const uint32_t grid = (p.nrb * p.ns + 7) / 8 * 8 * p.ncb;  // XCD-aware order; surplus workgroups exit
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * NW), lds, stream, p);
     return hipGetLastError();
 }
 
-// Rounds of resident workgroups times rows per workgroup: the planner's cost
-// of a row-tile count (the work of one round grows with NRT).
-template <int META, int NRT>
-double wide_cost(const WideParams &p, const DeviceLimits &lim) {
-    const uint32_t nrb = (p.rows + 16 * NRT - 1) / (16 * NRT);
-    const uint32_t per_cu = resident_per_cu(reinterpret_cast<const void *>(wide_mfma_kernel<META, NRT>),
-                                            wide_lds_bytes<META>(NRT));
-    const uint32_t slots = per_cu * uint32_t(std::max(lim.num_cus, 1));
-    const uint32_t wgs = nrb * p.ntb;
-    return double((wgs + slots - 1) / slots) * NRT * per_cu;
+// Centring costs 5% with two RHS tiles, where unpacking no longer hides under
+// the matrix cores (17408x5120, Q4, 128 RHS: 80.7 us, 76.7 without). Q4 does
+// without it there in group 32, and in group 64 with whole 256-column rows;
+// the other shapes' error was lower before (1.8e-7) and they are centred.
+template <int BITS, int META, bool G32>
+hipError_t launch_tile(const WideParams &p, const WidePlan &pl, hipStream_t stream) {
+#define QMR_WIDE(RT, CT, NW)                                                                                       \
+    if (pl.rt == RT && pl.ct == CT && pl.nw == NW) {                                                               \
+        if constexpr (BITS == 4 && CT == 2)                                                                        \
+            if (G32 || (p.group == 64 && p.cols % 256 == 0))                                                       \
+                return launch_instance<BITS, META, G32, false, RT, CT, NW>(p, stream);                             \
+        if constexpr (BITS == 8 || CT == 1 || !G32) return launch_instance<BITS, META, G32, true, RT, CT, NW>(p, stream); \
+    }
+    QMR_WIDE(2, 1, 8) QMR_WIDE(4, 1, 4) QMR_WIDE(4, 1, 8) QMR_WIDE(5, 1, 8) QMR_WIDE(8, 1, 8) QMR_WIDE(8, 1, 4)
+    QMR_WIDE(4, 2, 4) QMR_WIDE(4, 2, 8) QMR_WIDE(5, 2, 8) QMR_WIDE(7, 2, 4) QMR_WIDE(8, 2, 4)
+#undef QMR_WIDE
+    return hipErrorNotSupported;
 }
 
-template <int META>
-hipError_t launch_meta(const WideParams &p, const DeviceLimits &lim, hipStream_t stream) {
-    if (wide_lds_bytes<META>(17) <= lim.max_lds_per_block && wide_cost<META, 17>(p, lim) <= wide_cost<META, 8>(p, lim))
-        return launch_nrt<META, 17>(p, stream);
-    if (wide_lds_bytes<META>(8) > lim.max_lds_per_block) return hipErrorNotSupported;
-    return launch_nrt<META, 8>(p, stream);
+// Regions of the workspace.
+struct Regions {
+    size_t expo, planes, total;
+};
+Regions regions(const AffineArgs &a, const WidePlan &pl) {
+    auto up = [](size_t v) { return (v + 255) / 256 * 256; };
+    const size_t units = (a.cols + kUnit - 1) / kUnit, ntb = (a.batch + kRhsBlock - 1) / kRhsBlock;
+    Regions r{};
+    r.expo = up(units * ntb * kImgBytes);
+    r.planes = r.expo + up(size_t(pl.ns) * pl.nw * ntb * kRhsBlock * 4);
+    r.total = r.planes + (pl.ns > 1 ? size_t(pl.ns) * a.batch * a.rows * 4 : 0);
+    return r;
 }
 
 }  // namespace
 
 bool wide_mfma_supported(const AffineArgs &a) {
-    if (a.bits != 4 || a.group != 64) return false;
-    if (a.meta != Meta::F32 && a.meta != Meta::BF16) return false;
-    if (a.batch < 1 || a.batch > 256) return false;
-    if (a.cols % 256 != 0) return false;  // whole quads of groups (metadata items)
-    const uintptr_t al = reinterpret_cast<uintptr_t>(a.w) | reinterpret_cast<uintptr_t>(a.s) |
-                         reinterpret_cast<uintptr_t>(a.b);
-    // 32-bit buffer offsets: codes reach one workgroup's rows plus a row
-    // past the matrix, images and prefetches up to a chunk plus a quad of
-    // groups past the last one (all read as zeros).
-    const uint64_t w_span = (uint64_t(a.rows) + 16 * 17 + 2) * a.cols / 2;
+    if (a.bits != 4 && a.bits != 8) return false;
+    if (a.group != 32 && a.group != 64 && a.group != 128) return false;
+    if (a.batch < 1 || a.batch > 256 || a.residual || a.up_w) return false;
+    // 32-bit buffer offsets: codes reach one workgroup's rows past the
+    // matrix, images one chunk of units past the row (all read as zeros).
+    const uint64_t row_bytes = uint64_t(a.cols) * a.bits / 8;
     const uint64_t ntb = (a.batch + kRhsBlock - 1) / kRhsBlock;
-    const uint64_t img = (uint64_t(a.cols / 64) + kCG + 8) * ntb * kImgBytes;
-    return al % 16 == 0 && uint64_t(a.batch) * a.cols * 4 < (1ull << 31) && w_span < (1ull << 31) &&
-           img < (1ull << 31);
+    const uint64_t img = (uint64_t(a.cols + kUnit - 1) / kUnit + 40) * ntb * kImgBytes;
+    const uint64_t meta = uint64_t(a.rows) * (a.cols / a.group) * (a.meta == Meta::F32 ? 4 : 2);
+    return uint64_t(a.batch) * a.cols * 4 < (1ull << 31) && (uint64_t(a.rows) + 16 * 10) * row_bytes < (1ull << 31) &&
+           img < (1ull << 31) && meta < (1ull << 31) && meta >= 32;
 }
 
-size_t wide_mfma_workspace(const AffineArgs &a) {
-    const size_t ntb = (a.batch + kRhsBlock - 1) / kRhsBlock;
-    return size_t(a.cols / 64) * ntb * kImgBytes;
+// The plan is the cheapest of the compiled instances and up to eight K splits
+// under a model of what a workgroup does, fitted to 1500 timings (17 shapes
+// from 1024x1024 to 17408x5120, 4 to 256 RHS, both code sizes, groups 32, 64
+// and 128; its choice is on average 2.6% slower than the fastest plan, and
+// what is furthest off, 1.4x, are 200 RHS over 900 rows).
+WidePlan plan_wide(const AffineArgs &a, const DeviceLimits &lim, const WidePlan &force) {
+    struct Instance {
+        uint32_t rt, ct, nw, per_cu;  // per_cu: workgroups that fit a CU (LDS, registers)
+    };
+    constexpr Instance instances[] = {{2, 1, 8, 1}, {4, 1, 4, 3}, {4, 1, 8, 1}, {5, 1, 8, 1}, {8, 1, 8, 1}, {8, 1, 4, 2},
+                                      {4, 2, 4, 2}, {4, 2, 8, 1}, {5, 2, 8, 1}, {7, 2, 4, 2}, {8, 2, 4, 2}};
+    // Microseconds: a call, a group's products per row tile (one or two RHS
+    // tiles), the rest of a group step, a metadata chunk, the factor of a CU
+    // with less than two waves per SIMD, a round of workgroups, the sum launch
+    // and its planes per million floats.
+    constexpr float kCall = 6.67f, kStep[2] = {0.091f, 0.133f}, kFix = 0.271f, kChunk = 0.252f, kLone = 1.685f,
+                    kRound = 2.9f, kSum = 6.8f, kPlane = 1.6f;
+    const uint32_t units = (a.cols + kUnit - 1) / kUnit, nct = (a.batch + 15) / 16;
+    const uint32_t steps = a.group == 32 ? 4 : 2;  // group steps per unit
+    const uint32_t cus = uint32_t(std::max(lim.num_cus, 1));
+    auto split = [&](WidePlan pl) {
+        pl.ups = ((units + pl.ns - 1) / pl.ns + pl.nw - 1) / pl.nw * pl.nw;
+        pl.ns = (units + pl.ups - 1) / pl.ups;
+        return pl;
+    };
+    WidePlan best;
+    float best_us = 0.f;
+    for (const Instance &in : instances) {
+        if ((force.rt && force.rt != in.rt) || (force.ct && force.ct != in.ct) || (force.nw && force.nw != in.nw)) continue;
+        for (const uint32_t ns : {1u, 2u, 3u, 4u, 6u, 8u}) {
+            WidePlan pl;
+            pl.rt = in.rt;
+            pl.ct = in.ct;
+            pl.nw = in.nw;
+            pl.ns = force.ns ? force.ns : ns;
+            pl = split(pl);
+            // A split's classes all have a unit; its planes fit the scratch of
+            // the encode that allocates nothing, so that both take one plan.
+            if (!force.ns && ns > 1 && (units / ns < in.nw || regions(a, pl).total > QMR_STATIC_SCRATCH_BYTES)) continue;
+            const uint32_t upw = pl.ups / pl.nw;
+            const uint32_t wgs = (a.rows + 16 * in.rt - 1) / (16 * in.rt) * ((nct + in.ct - 1) / in.ct) * pl.ns;
+            const uint32_t k = (wgs + cus - 1) / cus;  // workgroups on the busiest CU
+            const float unit = float(steps * in.rt) * kStep[in.ct - 1] * (a.group == 32 ? 0.62f : 1.f) + kFix;
+            float us = float(k) * float(in.nw) / 4.f *
+                       (float(upw) * unit + float((upw * steps + 3) / 4) * kChunk);
+            if (std::min(k, in.per_cu) * in.nw < 8) us *= kLone;
+            us += kCall + float((k + in.per_cu - 1) / in.per_cu) * kRound;
+            if (pl.ns > 1) us += kSum + float(a.batch) * float(a.rows) * float(pl.ns) * kPlane * 1e-6f;
+            if (best.rt == 0 || us < best_us) best = pl, best_us = us;
+        }
+    }
+    return best;
 }
+
+size_t wide_mfma_workspace(const AffineArgs &a, const WidePlan &pl) { return regions(a, pl).total; }
 
 WideExtent wide_address_extent(uint32_t rows, uint32_t cols, uint32_t n, uint32_t nrt) {
     WideExtent out{};
-    const uint32_t G = cols / 64, nch = (G + kCG - 1) / kCG, ntb = (n + kRhsBlock - 1) / kRhsBlock;
+    const uint32_t units = (cols + kUnit - 1) / kUnit, ntb = (n + kRhsBlock - 1) / kRhsBlock;
     const uint32_t nrb = (rows + 16 * nrt - 1) / (16 * nrt);
-    const WideAddr A{rows, G, ntb, cols / 2};
+    const WideAddr A{rows, units, ntb, cols / 2};
     out.code_extent = uint64_t(rows) * cols / 2;
-    out.image_extent = uint64_t(G) * ntb * kImgBytes;
+    out.image_extent = uint64_t(units) * ntb * kImgBytes;
     auto note = [](uint64_t &mx, uint32_t v, uint32_t so, uint32_t size) {
         if (v != kOut) mx = std::max(mx, uint64_t(v) + so + size);
     };
-    // Groups the kernel requests per class kr: the first (kr) and, for each
-    // group it processes (16c + kr + 4i, c < nch, i < 4), the one four
-    // groups on (codes and x fragments alike); group sums per chunk c <= nch.
-    for (uint32_t kr = 0; kr < uint32_t(kKRanges); ++kr) {
-        for (uint32_t j = 0; j <= 4 * nch; ++j) {
-            const uint32_t g = kr + 4 * j;
-            for (uint32_t rb = 0; rb < nrb; ++rb)
-                for (uint32_t rt = 0; rt < nrt; ++rt)
-                    for (uint32_t l = 0; l < 64; ++l)
-                        note(out.code_end, A.code_v(rb * 16 * nrt, rt, l & 15, l >> 4, g), A.code_s(rt, g), 8);
-            for (uint32_t tb = 0; tb < ntb; ++tb)
-                for (uint32_t f = 0; f < 8; ++f)
-                    for (uint32_t l = 0; l < 64; ++l) note(out.image_end, A.frag_v(l, g), A.frag_s(g, tb, f), 16);
-        }
-        for (uint32_t c = 0; c <= nch; ++c)
-            for (uint32_t tb = 0; tb < ntb; ++tb)
+    // Every unit, and those past the row that the prefetches reach.
+    for (uint32_t u = 0; u < units + 32; ++u) {
+        for (uint32_t rb = 0; rb < nrb; ++rb)
+            for (uint32_t rt = 0; rt < nrt; ++rt)
                 for (uint32_t l = 0; l < 64; ++l)
-                    for (uint32_t ct = 0; ct < 2; ++ct)
-                        note(out.image_end, A.sum_v(c * kCG + kr, l >> 4, l & 15, ct), A.sum_s(c * kCG + kr, tb), 4);
+                    note(out.code_end, A.code_v(rb * 16 * nrt, rt, l >> 2, l & 3, u), A.code_s(rt, u), 16);
+        // RHS tiles up to a block of four past the images.
+        for (uint32_t ct = 0; ct < 2 * ntb + 4; ++ct)
+            for (uint32_t l = 0; l < 64; ++l) {
+                for (uint32_t f = 0; f < 8; ++f) note(out.image_end, A.frag_v(l, u, ct), A.frag_s(u, ct, f), 16);
+                for (uint32_t sub = 0; sub < 4; ++sub) note(out.image_end, A.sum_at(u, sub, ct, l & 15), 0, 4);
+            }
     }
     return out;
 }
 
-hipError_t launch_wide_mfma(const AffineArgs &a, unsigned char *workspace, const DeviceLimits &lim,
-                            hipStream_t stream) {
+hipError_t launch_wide_mfma(const AffineArgs &a, const WidePlan &pl, unsigned char *workspace, hipStream_t stream) {
+    const Regions r = regions(a, pl);
     WideParams p;
     p.w = a.w;
     p.s = a.s;
     p.b = a.b;
     p.x = a.x;
-    p.y = a.y;
     p.img = workspace;
+    p.expo = reinterpret_cast<int *>(workspace + r.expo);
+    float *planes = reinterpret_cast<float *>(workspace + r.planes);
+    p.y = pl.ns > 1 ? planes : a.y;
+    p.plane = pl.ns > 1 ? a.batch * a.rows : 0;
     p.rows = a.rows;
     p.cols = a.cols;
     p.n = a.batch;
+    p.group = a.group;
+    p.units = (a.cols + kUnit - 1) / kUnit;
+    p.groups = a.cols / a.group;
     p.ntb = (a.batch + kRhsBlock - 1) / kRhsBlock;
-    p.nrb = 0;
-    p.w_bytes = uint32_t(uint64_t(a.rows) * a.cols / 2);
-    p.m_bytes = uint32_t(uint64_t(a.rows) * (a.cols / 64) * (a.meta == Meta::F32 ? 4 : 2));
-    p.img_bytes = uint32_t(wide_mfma_workspace(a));
-    hipLaunchKernelGGL(wide_prep_kernel, dim3(a.cols / 64, p.ntb), dim3(kPrepThreads), 0, stream, p);
+    p.ncb = ((a.batch + 15) / 16 + pl.ct - 1) / pl.ct;
+    p.nrb = (a.rows + 16 * pl.rt - 1) / (16 * pl.rt);
+    p.ns = pl.ns;
+    p.ups = pl.ups;
+    p.w_bytes = uint32_t(uint64_t(a.rows) * a.cols * a.bits / 8);
+    p.m_bytes = uint32_t((uint64_t(a.rows) * p.groups * (a.meta == Meta::F32 ? 4 : 2) + 3) / 4 * 4);
+    p.img_bytes = uint32_t(size_t(p.units) * p.ntb * kImgBytes);
+    const uint32_t grid = 2 * p.ntb * pl.ns * pl.nw;
+    if (a.bits == 4)
+        hipLaunchKernelGGL(wide_prep_kernel<4>, dim3(grid), dim3(kPrepThreads), 0, stream, p, pl.nw);
+    else
+        hipLaunchKernelGGL(wide_prep_kernel<8>, dim3(grid), dim3(kPrepThreads), 0, stream, p, pl.nw);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    return a.meta == Meta::F32 ? launch_meta<0>(p, lim, stream) : launch_meta<1>(p, lim, stream);
+    const bool g32 = a.group == 32;
+    if (a.bits == 4)
+        e = a.meta == Meta::F32    ? (g32 ? launch_tile<4, 0, true>(p, pl, stream) : launch_tile<4, 0, false>(p, pl, stream))
+            : a.meta == Meta::BF16 ? (g32 ? launch_tile<4, 1, true>(p, pl, stream) : launch_tile<4, 1, false>(p, pl, stream))
+                                   : (g32 ? launch_tile<4, 2, true>(p, pl, stream) : launch_tile<4, 2, false>(p, pl, stream));
+    else
+        e = a.meta == Meta::F32    ? (g32 ? launch_tile<8, 0, true>(p, pl, stream) : launch_tile<8, 0, false>(p, pl, stream))
+            : a.meta == Meta::BF16 ? (g32 ? launch_tile<8, 1, true>(p, pl, stream) : launch_tile<8, 1, false>(p, pl, stream))
+                                   : (g32 ? launch_tile<8, 2, true>(p, pl, stream) : launch_tile<8, 2, false>(p, pl, stream));
+    if (e != hipSuccess || pl.ns == 1) return e;
+    const uint32_t count = a.batch * a.rows;
+    hipLaunchKernelGGL(wide_sum_kernel, dim3(std::min((count + 255) / 256, 2048u)), dim3(256), 0, stream, planes, a.y,
+                       count, pl.ns);
+    return hipGetLastError();
 }
 
 }  // namespace qmr

@@ -1,0 +1,58 @@
+"""Every workgroup shape of the wide kernel, in the formats it takes, at ragged
+rows, columns and RHS counts, against the FP64 oracle and, bit for bit, between
+qmr_encode and qmr_encode_static."""
+import os
+
+import numpy as np
+import pytest
+
+import oracle
+import qmr.synth as synth
+from helpers import upload_matrix
+
+pytestmark = pytest.mark.gpu
+THREADS = min(16, os.cpu_count() or 1)
+NAME = {"bf16": "_bf16", "f32": ""}
+# (row tiles, RHS tiles, waves) of 16, each with the K splits it is run with.
+SHAPES = [(0, 0, 0, 0), (2, 1, 8, 1), (4, 1, 4, 2), (4, 1, 8, 1), (5, 1, 8, 1), (8, 1, 8, 1), (8, 1, 4, 3),
+          (4, 2, 4, 2), (4, 2, 8, 1), (5, 2, 8, 1), (7, 2, 4, 1), (8, 2, 4, 2)]
+
+
+# One row more than whole tiles; a last unit of 32, 64 or 128 columns; odd group
+# counts (a BF16 row that starts inside a word); one RHS more than a tile or an
+# image; a matrix of fewer groups than a metadata window's.
+@pytest.mark.parametrize("rows,cols,bits,group,meta,batch",
+                         [(129, 1056, 4, 32, "bf16", 33), (65, 864, 8, 32, "f32", 17), (81, 1088, 4, 64, "bf16", 5),
+                          (257, 1024, 4, 64, "f32", 70), (113, 1984, 8, 64, "bf16", 256), (145, 1408, 4, 128, "bf16", 16),
+                          (33, 640, 8, 128, "f32", 34), (17, 64, 4, 64, "bf16", 6), (8, 128, 8, 128, "f32", 18)])
+def test_wide_shapes_and_formats(gpu, rows, cols, bits, group, meta, batch):
+    rng = np.random.default_rng(rows * cols + batch)
+    top = 2**bits
+    w = rng.integers(0, 2**32, rows * cols * bits // 32, dtype=np.uint32)
+    sf = rng.uniform(0.002, 0.02, rows * cols // group).astype(np.float32)
+    bf = (-top / 2 * sf + rng.normal(0, 1e-3, sf.size)).astype(np.float32)
+    s, b = (synth.f32_to_bf16_bits(sf), synth.f32_to_bf16_bits(bf)) if meta == "bf16" else (sf, bf)
+    x = (rng.standard_normal((batch, cols)) * np.exp2(rng.integers(-12, 13, (batch, 1)))).astype(np.float32)
+    want = oracle.matmul_f64(w, s, b, meta, x, rows, cols, bits, group, batch, THREADS).reshape(batch, rows)
+    # x in two halves is good to 2^-22, and no sum passes A = sum |x| (|s| top
+    # + |b|); a group makes at most 2 * group / 32 products, the scaling and
+    # the bias, each rounded to 2^-24 of A, and 32 more join classes and splits.
+    per = (np.repeat(np.abs(sf), group) * top + np.repeat(np.abs(bf), group)).reshape(rows, cols) * 1.01
+    bound = (2.0**-21 + (cols / group * (group / 16 + 3) + 32) * 2.0**-24) * (np.abs(x).astype(np.float64) @ per.T)
+    buffers = [*upload_matrix(gpu, w, s, b), gpu.upload_f32(x.ravel()), gpu.alloc_f32(batch * rows)]
+    name, params = "matmul_affine_wide" + NAME[meta], [rows, cols, bits, group, batch]
+    try:
+        for rt, ct, nw, ns in SHAPES:
+            print(f"shape {rt} {ct} {nw} splits {ns}", flush=True)
+            gpu.set_gemv_plan(-6, nw * 100000 + ns * 1000 + ct * 100 + rt)
+            gpu.dispatch(name, buffers, params)
+            assert gpu.last_hip_kernel().startswith("wide_mfma_kernel")
+            got = gpu.read_f32(buffers[4], batch * rows)
+            excess = np.abs(got.reshape(batch, rows) - want) / bound
+            assert excess.max() <= 1, f"shape {rt} {ct} {nw} splits {ns}: {excess.max():.2f} of the bound"
+            command = gpu.begin()
+            command.encode(name, buffers, params, rows * 32, 64, static_scratch=True)
+            command.finish()
+            assert np.array_equal(gpu.read_f32(buffers[4], batch * rows), got), "encode_static differs"
+    finally:
+        gpu.set_gemv_plan(0, 0)
