@@ -683,12 +683,48 @@ hipError_t launch_dense(qmr_device *dev, const uint16_t *w, const float *x, floa
     return e;
 }
 
+// The wide kernel with its images (and the planes of K splits) in the
+// device's workspace or, for qmr_encode_static, in the static scratch.
+hipError_t launch_wide(qmr_device *dev, const qmr::AffineArgs &a, const qmr::WidePlan &pl, unsigned char *fixed) {
+    const size_t need = qmr::wide_mfma_workspace(a, pl);
+    if (fixed) {
+        check_static_scratch(need, "wide-block activation images");
+        mark_static_dirty(dev, need);
+    } else if (need > dev->ws_wide_bytes) {
+        check_hip(hipStreamSynchronize(dev->stream), "hipStreamSynchronize");
+        if (dev->ws_wide) hipFree(dev->ws_wide);
+        dev->ws_wide = nullptr;
+        dev->ws_wide_bytes = 0;
+        check_hip(hipMalloc(&dev->ws_wide, need), "hipMalloc (wide workspace)");
+        dev->ws_wide_bytes = need;
+    }
+    dev->last_hip = "wide_mfma_kernel";
+    start_gpu(dev);
+    return qmr::launch_wide_mfma(a, pl, fixed ? fixed : dev->ws_wide, dev->stream);
+}
+
+// Blocks of three and four RHS in group 32, which the other matrix-core
+// kernels don't take, on the wide kernel instead of the vector-ALU one: where
+// the block's x no longer fits a workgroup's LDS (900x13312 Q4, four RHS: 54
+// us against 15), and, for matrices of more than one round of workgroups,
+// where it leaves room for one or two workgroups per CU (9001x4160 Q4, four
+// RHS: 26.6 us against 19.9; 17408x5120: 51 against 26; Q8 68 against 37).
+// Below the lines the vector-ALU kernel wins: 4096x5120 with four RHS 14.0 us
+// against 14.5, 10000x5120 with three 18.0 against 20.0, 9001x4160 Q8 20.1
+// against 23.4, and small matrices have no use for two launches (1024x1024:
+// 3.5 us against 8.3).
+bool wide_block_preferred(const qmr::AffineArgs &a) {
+    if (a.group != 32 || a.batch < 3) return false;
+    const uint64_t x = uint64_t(a.batch) * a.cols;
+    return x > 36864 || (a.rows >= 7000 && x >= (a.bits == 4 ? 16384u : 20480u));
+}
+
 // One packed-affine product of at most four RHS: the row-band matrix-core
 // kernel where it has a plan whose workgroups are all resident at once; else
 // the split-K matrix-core kernel where it supports the format, unless
 // rows_preferred() hands the shape to the row-owning matrix-core kernel;
-// else the vector-ALU kernels. A forced plan (testing hook) of rr > 0 or
-// rr == -1 selects the vector-ALU tilings, rr == -4 the row-band kernel,
+// else the wide kernel (wide_block_preferred()) or the vector-ALU kernels. A
+// forced plan (testing hook) of rr > 0 or rr == -1 selects the vector-ALU tilings, rr == -4 the row-band kernel,
 // rr == -3 the row-owning matrix-core kernel, rr == -2 the split-K kernel
 // whatever its shape (with ks > 0 splits, when that count is feasible).
 // `fixed` (qmr_encode_static) puts every workspace in the static scratch.
@@ -722,6 +758,10 @@ hipError_t launch_product(qmr_device *dev, const qmr::AffineArgs &a, unsigned ch
             dev->last_hip = "affine_mfma_kernel";
             return launch_split_k(dev, a, pl, fixed);
         }
+    }
+    if (f.rr == 0 && wide_block_preferred(a) && qmr::wide_mfma_supported(a)) {
+        const qmr::WidePlan pl = qmr::plan_wide(a, dev->limits);
+        if (!fixed || qmr::wide_mfma_workspace(a, pl) <= QMR_STATIC_SCRATCH_BYTES) return launch_wide(dev, a, pl, fixed);
     }
     // The vector-ALU kernels have no fused epilogue.
     ensure(a.residual == nullptr, "fused product needs a matrix-core kernel", QMR_ERR_UNSUPPORTED);
@@ -1337,24 +1377,7 @@ static int encode_command(qmr_command *command, const char *cname, qmr_buffer *c
                 }
             }
             if (wpl.rt > 0) {
-                const size_t need = qmr::wide_mfma_workspace(a, wpl);
-                unsigned char *images = fixed;
-                if (fixed) {
-                    check_static_scratch(need, "wide-block activation images");
-                    mark_static_dirty(dev, need);
-                }
-                if (!fixed && need > dev->ws_wide_bytes) {
-                    check_hip(hipStreamSynchronize(dev->stream), "hipStreamSynchronize");
-                    if (dev->ws_wide) hipFree(dev->ws_wide);
-                    dev->ws_wide = nullptr;
-                    dev->ws_wide_bytes = 0;
-                    check_hip(hipMalloc(&dev->ws_wide, need), "hipMalloc (wide workspace)");
-                    dev->ws_wide_bytes = need;
-                }
-                if (!fixed) images = dev->ws_wide;
-                dev->last_hip = "wide_mfma_kernel";
-                start_gpu(dev);
-                e = qmr::launch_wide_mfma(a, wpl, images, dev->stream);
+                e = launch_wide(dev, a, wpl, fixed);
             } else if (wide) {
                 // Up to four RHS and what the wide kernel doesn't take:
                 // successive blocks of up to four RHS.

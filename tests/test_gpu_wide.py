@@ -56,3 +56,35 @@ def test_wide_shapes_and_formats(gpu, rows, cols, bits, group, meta, batch):
             assert np.array_equal(gpu.read_f32(buffers[4], batch * rows), got), "encode_static differs"
     finally:
         gpu.set_gemv_plan(0, 0)
+
+
+# On both sides of the lines in rows, in columns and in RHS count.
+@pytest.mark.parametrize("rows,cols,bits,batch,wide", [(7001, 4096, 4, 4, True), (6999, 4096, 4, 4, False),
+                                                       (7000, 4064, 4, 4, False), (7000, 5120, 8, 4, True),
+                                                       (7000, 5088, 8, 4, False), (17, 12320, 4, 3, True),
+                                                       (17, 12288, 8, 3, False), (40, 9248, 8, 4, True),
+                                                       (7000, 20480, 4, 2, False)])
+def test_group_32_blocks_on_either_kernel(gpu, rows, cols, bits, batch, wide):
+    """The default route of a group 32 block and the vector-ALU kernel agree to
+    the bounds of both: four FP32 roundings for each column at the very most."""
+    rng = np.random.default_rng(rows + cols)
+    top = 2**bits
+    w = rng.integers(0, 2**32, rows * cols * bits // 32, dtype=np.uint32)
+    s = rng.uniform(0.002, 0.02, rows * cols // 32).astype(np.float32)
+    b = (-top / 2 * s + rng.normal(0, 1e-3, s.size)).astype(np.float32)
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    buffers = [*upload_matrix(gpu, w, s, b), gpu.upload_f32(x.ravel()), gpu.alloc_f32(batch * rows)]
+    got = []
+    try:
+        for plan in ((0, 0), (-1, 0)):
+            print(f"plan {plan}", flush=True)
+            gpu.set_gemv_plan(*plan)
+            gpu.dispatch("matmul_affine", buffers, [rows, cols, bits, 32, batch])
+            if plan == (0, 0):
+                assert (gpu.last_hip_kernel() == "wide_mfma_kernel") == wide
+            got.append(gpu.read_f32(buffers[4], batch * rows).reshape(batch, rows).astype(np.float64))
+    finally:
+        gpu.set_gemv_plan(0, 0)
+    per = (np.repeat(s, 32) * top + np.repeat(np.abs(b), 32)).reshape(rows, cols)
+    bound = 4 * cols * 2.0**-24 * (np.abs(x).astype(np.float64) @ per.T.astype(np.float64))
+    assert (np.abs(got[0] - got[1]) <= bound).all()
