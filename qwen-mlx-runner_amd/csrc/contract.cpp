@@ -13,9 +13,12 @@ namespace {
 
 [[noreturn]] void fail(const std::string &message) { throw Error{1, message}; }
 
-void ensure(bool ok, const std::string &message) {
-    if (!ok) fail(message);
-}
+// A macro, so that the message is put together only where the check fails:
+// every encode makes these checks.
+#define ensure(ok, ...)              \
+    do {                             \
+        if (!(ok)) fail(__VA_ARGS__); \
+    } while (0)
 
 bool mul_overflow(size_t a, size_t b, size_t *out) { return __builtin_mul_overflow(a, b, out); }
 

@@ -143,9 +143,15 @@ int guarded(F &&f) {
     }
 }
 
-void ensure(bool ok, const std::string &message, int code = QMR_ERR_INVALID) {
-    if (!ok) throw Error{code, message};
-}
+[[noreturn]] void fail(const std::string &message, int code = QMR_ERR_INVALID) { throw Error{code, message}; }
+
+// A macro, so that the message is put together only where the check fails: the
+// strings of about 40 checks cost 1 us of every encode (96 embedding rows: 726
+// us a pass with them, 629 without).
+#define ensure(ok, ...)              \
+    do {                             \
+        if (!(ok)) fail(__VA_ARGS__); \
+    } while (0)
 
 void check_hip(hipError_t e, const char *what) {
     if (e != hipSuccess) throw Error{QMR_ERR_DEVICE, std::string(what) + ": " + hipGetErrorString(e)};
