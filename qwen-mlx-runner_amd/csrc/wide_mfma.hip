@@ -5,7 +5,8 @@
 //     D[r,t,g] = sum_{c in g} q[r,c] * x[t,c],  S[t,g] = sum_{c in g} x[t,c].
 // D runs on v_mfma_f32_16x16x32_f16 with exact integer codes (f16 subnormals,
 // as in mfma_common.hpp, or centred ones) against x split into hi/lo f16 parts, so it is
-// accurate to about 2^-22; the scales multiply D in FP32 and the bias term is
+// accurate to about 2^-22, or, in group 32, on v_mfma_f32_16x16x32_bf16 against
+// the three bf16 parts of x, which are all of it; the scales multiply D in FP32 and the bias term is
 // an FP32 matrix product of S and b (v_mfma_f32_16x16x4_f32 over four groups
 // at a time).
 //
@@ -50,6 +51,7 @@ using namespace mfma;
 typedef uint32_t u2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u3 __attribute__((ext_vector_type(3)));
 typedef int i4 __attribute__((ext_vector_type(4)));
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 
 // Codes as f16: Q4 as subnormals (the code times 2^-20), Q8 as 1024 + code;
 // centred, less the middle of their range (8 or 128), which goes into the
@@ -76,13 +78,53 @@ __device__ __forceinline__ h8 wide_unpack(const u2 &w) {
     }
 }
 
+// Group 32: codes as bf16, centred, against x in three bf16 parts, which hold
+// all 24 bits of an FP32 value over its whole range: such blocks ran on the
+// vector ALU, which multiplies FP32 values, and in fewer bits a token's small
+// columns would be lost beside its large ones. Error against 64 bits at 5120
+// columns 1.5e-7 (Q4) and 1.4e-7 (Q8), on the vector ALU 2.5e-7 and 2.0e-7;
+// with one column 1e4 times the others 1.8e-7 and 1.7e-7 (Q4 in two f16 parts
+// 9e-7). The third part costs 10% at 4 RHS and 24-35% from 64 RHS on.
+template <int BITS>
+__device__ __forceinline__ u4 bf16_codes(const u2 &w) {
+    auto pair = [](float lo, float hi) {  // exact: at most eight bits each
+        return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+    };
+    if constexpr (BITS == 4) {  // sixteenths
+        const uint32_t even = w.x ^ 0x88888888u, odd = even >> 4;
+        auto f = [](uint32_t v) { return __builtin_amdgcn_cvt_off_f32_i4(int(v)); };
+        return u4{pair(f(even), f(odd)), pair(f(even >> 8), f(odd >> 8)), pair(f(even >> 16), f(odd >> 16)),
+                  pair(f(even >> 24), f(odd >> 24))};
+    } else {
+        const uint32_t x = w.x ^ 0x80808080u, y = w.y ^ 0x80808080u;
+        auto f = [](uint32_t v, int k) { return float(int8_t(v >> (8 * k))); };
+        return u4{pair(f(x, 0), f(x, 1)), pair(f(x, 2), f(x, 3)), pair(f(y, 0), f(y, 1)), pair(f(y, 2), f(y, 3))};
+    }
+}
+// Factors of a group 32 x and of its scales: code * x is at most half of x, so
+// that a group's sum overflows where the sum of its x does, not before.
+template <int BITS>
+constexpr float kXFactor = BITS == 4 ? 1.f : 1.f / 256;
+template <int BITS>
+constexpr float kSFactor = BITS == 4 ? 16.f : 256.f;
+
+template <bool G32>
+__device__ __forceinline__ f4 product(const u4 &x, const u4 &codes, const f4 &c) {
+    if constexpr (G32)
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, x), __builtin_bit_cast(b8, codes), c, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, x), __builtin_bit_cast(h8, codes), c, 0, 0, 0);
+}
+
 constexpr int kPrepThreads = 1024;
 constexpr uint32_t kUnit = 128;                 // columns per unit: four K steps of the MFMA
-constexpr int kRhsBlock = 32;                   // RHS per image
+constexpr int kRhsBlock = 32;                   // RHS tiles come in pairs
 constexpr int kFragBytes = 1024;                // one MFMA A fragment (64 lanes x 16 B)
-constexpr int kImgS = 16 * kFragBytes;          // [quarter or half][32] f32 column sums
-constexpr int kImgBytes = 16896;                // image stride
-static_assert(kImgS + 4 * kRhsBlock * 4 <= kImgBytes, "image layout");
+// An image: one unit of one RHS tile. Its fragments [K step][part], then the
+// column sums [quarter (group 32) or half][16] f32.
+constexpr uint32_t parts_of(bool g32) { return g32 ? 3 : 2; }
+constexpr uint32_t img_sums(bool g32) { return 4 * parts_of(g32) * kFragBytes; }
+constexpr uint32_t img_bytes(bool g32) { return img_sums(g32) + 256; }
 
 // A wave's piece of LDS: codes on their way to operand order (64 bytes of each
 // row, one unit of Q4 or half a unit of Q8; rows 80 bytes apart so that
@@ -95,9 +137,10 @@ constexpr size_t code_bytes(int nrt) { return size_t(16) * nrt * kCodePitch; }
 constexpr int meta_pitch(int nw) { return 4 * nw + 2; }
 constexpr size_t meta_bytes(int nrt, int nw) { return size_t(16) * nrt * meta_pitch(nw) * 8; }
 constexpr int kRedPad = 16;  // words between row tiles of the final planes
+constexpr size_t kFlagBytes = 64;  // behind the planes: a word per wave and RHS tile
 constexpr size_t wide_lds_bytes(int nrt, int nct, int nw) {
     const size_t red = size_t(nw > 4 ? 4 : nw) * nrt * (nct * 256 + kRedPad) * 4;  // [plane][rt][ct][v][lane] f32
-    return std::max(2 * meta_bytes(nrt, nw) + nw * code_bytes(nrt), red);
+    return std::max(2 * meta_bytes(nrt, nw) + nw * code_bytes(nrt), red + kFlagBytes);
 }
 
 // Byte offsets of the contraction kernel's code, x-fragment and group-sum
@@ -110,7 +153,9 @@ constexpr size_t wide_lds_bytes(int nrt, int nct, int nw) {
 // soffset + size within its view. qmr_wide_address_extent walks these on the
 // host.
 struct WideAddr {
-    uint32_t rows, units, ntb, row_bytes;
+    uint32_t rows, units, tiles, row_bytes;  // tiles: RHS tiles with an image
+    uint32_t ntb;                            // pairs of RHS tiles
+    bool g32;
     // Lane (row16, piece) loads 16 bytes of row row0 + 16 rt + row16 at byte
     // 64 seg + 16 piece (a unit is one 64-byte segment of Q4, two of Q8).
     __host__ __device__ uint32_t code_v(uint32_t row0, uint32_t rt, uint32_t row16, uint32_t piece, uint32_t seg) const {
@@ -118,19 +163,18 @@ struct WideAddr {
                                                                                  : kOut;
     }
     __host__ __device__ uint32_t code_s(uint32_t rt, uint32_t seg) const { return rt * 16 * row_bytes + 64 * seg; }
-    // Fragment f = 2*ks + hl of RHS tile ct in unit u; lane l reads 16 bytes.
+    // Fragment f of RHS tile ct in unit u; lane l reads 16 bytes.
+    __host__ __device__ uint32_t image(uint32_t u, uint32_t ct) const { return (u * 2 * ntb + ct) * img_bytes(g32); }
     __host__ __device__ uint32_t frag_v(uint32_t lane, uint32_t u, uint32_t ct) const {
-        return u < units && ct < 2 * ntb ? lane * 16 : kOut;
+        return u < units && ct < tiles ? lane * 16 : kOut;
     }
     __host__ __device__ uint32_t frag_s(uint32_t u, uint32_t ct, uint32_t f) const {
-        return (u * ntb + (ct >> 1)) * uint32_t(kImgBytes) + ((ct & 1) * 8 + f) * uint32_t(kFragBytes);
+        return image(u, ct) + f * uint32_t(kFragBytes);
     }
     // Sum of RHS 16 ct + r16 over quarter `sub` of unit u (group 32) or half
     // `sub` (the other groups).
     __host__ __device__ uint32_t sum_at(uint32_t u, uint32_t sub, uint32_t ct, uint32_t r16) const {
-        return u < units && ct < 2 * ntb
-                   ? (u * ntb + (ct >> 1)) * uint32_t(kImgBytes) + uint32_t(kImgS) + sub * (kRhsBlock * 4) + (ct & 1) * 64 + r16 * 4
-                   : kOut;
+        return u < units && ct < tiles ? image(u, ct) + img_sums(g32) + sub * 64 + r16 * 4 : kOut;
     }
 };
 
@@ -140,8 +184,8 @@ struct WideParams {
     const void *b;
     const float *x;
     float *y;              // output, or the first K split's plane
-    unsigned char *img;    // [units][ntb] images of kImgBytes
-    int *expo;             // [ns * nw][32 ntb] exponents e of the images' 2^-e
+    unsigned char *img;    // [units][2 ntb] images
+    int *expo;             // [ns * nw][32 ntb] exponents e of the images' 2^-e (not group 32)
     uint32_t rows, cols, n;       // n = RHS count
     uint32_t group;
     uint32_t units, groups;       // 128-column units (the last may be partial) and quant groups per row
@@ -203,8 +247,8 @@ __global__ __launch_bounds__(kPrepThreads) void wide_prep_kernel(WideParams p, u
     const float sc = __uint_as_float(uint32_t(127 - e) << 23);
     if (tid < 16) p.expo[size_t(cls) * (kRhsBlock * p.ntb) + t] = e;
     auto store = [&](const float (&xv)[4][8], uint32_t u) {
-        unsigned char *img = p.img + (size_t(u) * p.ntb + (ct >> 1)) * kImgBytes;
-        unsigned char *frag = img + (ct & 1) * 8 * kFragBytes + lane * 16;
+        unsigned char *img = p.img + (size_t(u) * 2 * p.ntb + ct) * img_bytes(false);
+        unsigned char *frag = img + lane * 16;
         float quarter[4];  // this lane's part of the sum of each K step's 32 columns
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
@@ -220,23 +264,18 @@ __global__ __launch_bounds__(kPrepThreads) void wide_prep_kernel(WideParams p, u
             *reinterpret_cast<u4 *>(frag + 2 * ks * kFragBytes) = hw;
             *reinterpret_cast<u4 *>(frag + (2 * ks + 1) * kFragBytes) = lw;
         }
-        // Sums of the unit's quarters (group 32) or halves, with the codes'
-        // power of two, so that b * S adds to s * D.
+        // Sums of the unit's halves, with the codes' power of two, so that b *
+        // S adds to s * D.
         const float cs = sc * (1.f / float(1u << kWideExp<BITS>));
-        float *S = reinterpret_cast<float *>(img + kImgS) + (ct & 1) * 16 + t16;
+        float *S = reinterpret_cast<float *>(img + img_sums(false)) + t16;
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
             quarter[ks] += __shfl_xor(quarter[ks], 16);
             quarter[ks] += __shfl_xor(quarter[ks], 32);
         }
         if (c4 == 0) {
-            if (p.group == 32) {
-#pragma unroll
-                for (int ks = 0; ks < 4; ++ks) S[ks * kRhsBlock] = quarter[ks] * cs;
-            } else {
-                S[0] = (quarter[0] + quarter[1]) * cs;
-                S[kRhsBlock] = (quarter[2] + quarter[3]) * cs;
-            }
+            S[0] = (quarter[0] + quarter[1]) * cs;
+            S[16] = (quarter[2] + quarter[3]) * cs;
         }
     };
     if (first < u1) store(x0, first);
@@ -245,6 +284,74 @@ __global__ __launch_bounds__(kPrepThreads) void wide_prep_kernel(WideParams p, u
         load(xv, u);
         store(xv, u);
     }
+}
+
+// The images of group 32: a wave per unit and RHS tile, lane (t16, c4) as
+// above. Parts are cut off, not rounded: three times eight bits are all of a
+// value's, and the first does not overflow. Inf and NaN stay out of the
+// fragments; NaN in place of their quarter's sum says that there are some.
+constexpr uint32_t kPrep32Waves = 4;
+template <int BITS>
+__global__ __launch_bounds__(64 * kPrep32Waves) void wide_prep32_kernel(WideParams p, uint32_t tiles) {
+    const uint32_t i = blockIdx.x * kPrep32Waves + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const uint32_t u = i / tiles, ct = i % tiles;
+    if (u >= p.units) return;
+    const uint32_t t16 = lane & 15, c4 = lane >> 4, t = ct * 16 + t16;
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>(p.x), 0, int(p.n * p.cols * 4u), kRsrcWord3);
+    unsigned char *img = p.img + (size_t(u) * 2 * p.ntb + ct) * img_bytes(true);
+    float xv[4][8];
+#pragma unroll
+    for (uint32_t ks = 0; ks < 4; ++ks) load_x8(xv[ks], xr, t, u * kUnit + 32 * ks + 8 * c4, p.cols, t < p.n);
+#pragma unroll
+    for (uint32_t ks = 0; ks < 4; ++ks) {
+        float(&v)[8] = xv[ks];
+        float bad = 0.f;  // NaN where a value is not finite
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const bool finite = __builtin_isfinite(v[j]);
+            bad = finite ? bad : __builtin_nanf("");
+            v[j] = finite ? v[j] : 0.f;
+        }
+        float sum = bad + (((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7])));
+        sum += __shfl_xor(sum, 16);
+        sum += __shfl_xor(sum, 32);
+        if (c4 == 0) reinterpret_cast<float *>(img + img_sums(true))[ks * 16 + t16] = sum;
+        u4 part[3];
+#pragma unroll
+        for (int e2 = 0; e2 < 4; ++e2) {
+            float r0 = v[2 * e2] * kXFactor<BITS>, r1 = v[2 * e2 + 1] * kXFactor<BITS>;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const uint32_t b0 = __float_as_uint(r0) & 0xFFFF0000u, b1 = __float_as_uint(r1) & 0xFFFF0000u;
+                part[k][e2] = b0 >> 16 | b1;
+                r0 -= __uint_as_float(b0);
+                r1 -= __uint_as_float(b1);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 3; ++k) *reinterpret_cast<u4 *>(img + (3 * ks + k) * kFragBytes + lane * 16) = part[k];
+    }
+}
+
+// What Inf and NaN among the columns [c0, c1) of an RHS add to row r of a
+// group 32 product, as the vector-ALU kernel has it: code * x times the scale,
+// and the bias times x.
+template <int BITS, int META>
+__device__ float non_finite(const WideParams &p, uint32_t t, uint32_t c0, uint32_t c1, uint32_t r) {
+    constexpr uint32_t PACK = 32 / BITS;
+    float sum = 0.f;
+    for (uint32_t c = c0; c < c1; ++c) {
+        const float v = p.x[size_t(t) * p.cols + c];
+        if (__builtin_isfinite(v)) continue;
+        const uint32_t code = p.w[size_t(r) * (p.cols / PACK) + c / PACK] >> (c % PACK * BITS) & ((1u << BITS) - 1);
+        const size_t g = size_t(r) * p.groups + c / 32;
+        auto meta = [&](const void *m) {
+            return META == 0 ? static_cast<const float *>(m)[g] : meta_f32<META>(static_cast<const uint16_t *>(m)[g]);
+        };
+        sum += meta(p.s) * (float(code) * v) + meta(p.b) * v;
+    }
+    return sum;
 }
 
 // ---- 2. The contraction. Lane (r16, q) of a wave: row r16 of every row
@@ -256,6 +363,7 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
     constexpr int SEG = BITS / 4;         // 64-byte code segments per unit
     constexpr int KPS = 4 / SEG;          // K steps per segment
     constexpr int KG = G32 ? 1 : 2;       // K steps per group (or half of 128)
+    constexpr int PARTS = parts_of(G32);  // of x
     constexpr int SL = 4 / KG;            // slots (groups or halves of 128) per unit
     constexpr uint32_t UPC = 4 / SL;      // units per chunk: four slots, one bias product
     constexpr int THREADS = 64 * NW_, PITCH = meta_pitch(NW_);
@@ -277,7 +385,7 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
     const uint32_t rb = pair % p.nrb, split = pair / p.nrb;
     const uint32_t row0 = rb * ROWS, ct0 = cb * NCT;
     const uint32_t u0 = split * p.ups, u1 = min(u0 + p.ups, p.units);
-    const WideAddr A{p.rows, u1, p.ntb, p.cols / (32 / BITS) * 4};
+    const WideAddr A{p.rows, u1, G32 ? (p.n + 15) / 16 : 2 * p.ntb, p.cols / (32 / BITS) * 4, p.ntb, G32};
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint32_t *>(p.w), 0, int(p.w_bytes), kRsrcWord3);
     const __amdgpu_buffer_rsrc_t ir = __builtin_amdgcn_make_buffer_rsrc(p.img, 0, int(p.img_bytes), kRsrcWord3);
@@ -384,6 +492,7 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
             for (uint32_t k = 0; k < 8; ++k) {  // past the split's groups there may be a neighbour's
                 sv[k] = g + k < g_end ? sv[k] : 0.f;
                 bv[k] = g + k < g_end ? CENTRED ? __builtin_fmaf(middle_of(BITS), sv[k], bv[k]) : bv[k] : 0.f;
+                if constexpr (G32) sv[k] *= kSFactor<BITS>;
             }
             if (rl >= uint32_t(ROWS)) continue;
             // Unit NW*i + class of the chunk: slots 4*class + 2*i + half
@@ -413,15 +522,15 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
         }
     };
     // ---- x
-    u4 xf[4][NCT][2];  // a unit's K steps; whole words: halves carried across the loop would be taken apart and put together
-    auto load_x = [&](u4 (&dst)[NCT][2], uint32_t u, uint32_t ks) {
+    u4 xf[4][NCT][PARTS];  // a unit's K steps; whole words: halves carried across the loop would be taken apart and put together
+    auto load_x = [&](u4 (&dst)[NCT][PARTS], uint32_t u, uint32_t ks) {
 #pragma unroll
         for (int ct = 0; ct < NCT; ++ct) {
             const int v = int(A.frag_v(uint32_t(lane), u, ct0 + uint32_t(ct)));
 #pragma unroll
-            for (int hl = 0; hl < 2; ++hl)
-                dst[ct][hl] = __builtin_bit_cast(
-                    u4, __builtin_amdgcn_raw_buffer_load_b128(ir, v, int(A.frag_s(u, ct0 + uint32_t(ct), 2 * ks + uint32_t(hl))), 0));
+            for (int part = 0; part < PARTS; ++part)
+                dst[ct][part] = __builtin_bit_cast(
+                    u4, __builtin_amdgcn_raw_buffer_load_b128(ir, v, int(A.frag_s(u, ct0 + uint32_t(ct), PARTS * ks + uint32_t(part))), 0));
         }
     };
     // Bias A operands of chunk c: lane (t16, q) the sum of slot q.
@@ -435,6 +544,15 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
 
     f4 acc[NRT][NCT];
     float sa[NCT];
+    bool bad[NCT] = {};  // group 32: Inf or NaN in the columns of sa
+    auto clean = [&](float (&sop)[NCT]) {
+#pragma unroll
+        for (int ct = 0; ct < NCT; ++ct) {
+            const bool nan = sop[ct] != sop[ct];
+            bad[ct] |= nan;
+            sop[ct] = nan ? 0.f : sop[ct];
+        }
+    };
     {
         const uint32_t u = u0 + uint32_t(wv);
         MStage st;
@@ -486,7 +604,7 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
                     // products and, on the vector ALU, the epilogue of tile
                     // rt-1 and the unpacking of tile rt+1; codes and scales
                     // are read from LDS two tiles ahead.
-                    h8 op[2][KG];
+                    u4 op[2][KG];
                     u2 w[2][KG];
                     float sv[3];
                     auto fetch = [&](int rt) {
@@ -496,7 +614,10 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
                     };
                     auto open = [&](int rt) {
 #pragma unroll
-                        for (int k = 0; k < KG; ++k) op[rt & 1][k] = wide_unpack<BITS, CENTRED>(w[rt & 1][k]);
+                        for (int k = 0; k < KG; ++k) {
+                            if constexpr (G32) op[rt & 1][k] = bf16_codes<BITS>(w[rt & 1][k]);
+                            else op[rt & 1][k] = __builtin_bit_cast(u4, wide_unpack<BITS, CENTRED>(w[rt & 1][k]));
+                        }
                     };
                     f4 d[2][NCT];
                     auto close = [&](int rt) {
@@ -516,14 +637,13 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
                         // of hi and lo in turn (2.4e-7 against 4.4e-7 at 5120
                         // columns, Q4), a quarter of lo first.
 #pragma unroll
-                        for (int hl = 0; hl < 2; ++hl)
+                        for (int part = 0; part < PARTS; ++part)
 #pragma unroll
                             for (int k = 0; k < KG; ++k)
 #pragma unroll
                                 for (int ct = 0; ct < NCT; ++ct)
-                                    d[rt & 1][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                                        __builtin_bit_cast(h8, xf[ks + k][ct][hl]), op[rt & 1][k],
-                                        k == 0 && hl == 0 ? zero : d[rt & 1][ct], 0, 0, 0);
+                                    d[rt & 1][ct] = product<G32>(xf[ks + k][ct][part], op[rt & 1][k],
+                                                                 k == 0 && part == 0 ? zero : d[rt & 1][ct]);
                         if (rt + 1 < NRT) open(rt + 1);
                         if (rt > 0) close(rt - 1);
                         if (rt + 2 < NRT) fetch(rt + 2);
@@ -539,6 +659,7 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
             // unit: b * S cancels most of s * D, so in the middle the sums
             // stray half as far.
             if (h == 0) {
+                if constexpr (G32) clean(sa);
 #pragma unroll
                 for (int rt = 0; rt < NRT; ++rt) {
                     const float bv = mb[rt * 16 * PITCH + q];
@@ -562,16 +683,18 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
     float *red = reinterpret_cast<float *>(lds);
     constexpr int TILE = NCT * 256 + kRedPad;
     constexpr uint32_t PLANES = NW > 4 ? 4 : NW;
+    if constexpr (!G32) {
 #pragma unroll
-    for (int ct = 0; ct < NCT; ++ct) {
-        const uint32_t t = (ct0 + uint32_t(ct)) * 16 + uint32_t(q) * 4;
-        i4 e{0, 0, 0, 0};
-        if (ct0 + uint32_t(ct) < 2 * p.ntb)
-            e = *reinterpret_cast<const i4 *>(p.expo + size_t(split * NW + uint32_t(wv)) * (kRhsBlock * p.ntb) + t);
+        for (int ct = 0; ct < NCT; ++ct) {
+            const uint32_t t = (ct0 + uint32_t(ct)) * 16 + uint32_t(q) * 4;
+            i4 e{0, 0, 0, 0};
+            if (ct0 + uint32_t(ct) < 2 * p.ntb)
+                e = *reinterpret_cast<const i4 *>(p.expo + size_t(split * NW + uint32_t(wv)) * (kRhsBlock * p.ntb) + t);
 #pragma unroll
-        for (int rt = 0; rt < NRT; ++rt)
+            for (int rt = 0; rt < NRT; ++rt)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) acc[rt][ct][v] = ldexpf(acc[rt][ct][v], e[v] + kWideExp<BITS>);
+                for (int v = 0; v < 4; ++v) acc[rt][ct][v] = ldexpf(acc[rt][ct][v], e[v] + kWideExp<BITS>);
+        }
     }
     auto place = [&](int rt, int ct, int v) -> float & {
         return red[((wv % int(PLANES)) * NRT + rt) * TILE + (ct * 4 + v) * 64 + lane];
@@ -596,6 +719,19 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
         }
         lds_barrier();
     }
+    uint32_t inf[NCT] = {};  // RHS with Inf or NaN in this split, a bit each
+    if constexpr (G32) {
+        uint32_t *flags = reinterpret_cast<uint32_t *>(lds + wide_lds_bytes(NRT, NCT, NW_) - kFlagBytes);
+#pragma unroll
+        for (int ct = 0; ct < NCT; ++ct) {
+            const uint64_t b = __ballot(bad[ct]);
+            if (lane == 0) flags[wv * NCT + ct] = uint32_t(b | b >> 16 | b >> 32 | b >> 48) & 0xFFFFu;
+        }
+        lds_barrier();
+#pragma unroll
+        for (int ct = 0; ct < NCT; ++ct)
+            for (uint32_t k = 0; k < NW; ++k) inf[ct] |= flags[k * NCT + ct];
+    }
     float *out = p.y + size_t(split) * p.plane;
     const uint32_t rows_here = min(uint32_t(ROWS), p.rows - row0);
     for (uint32_t i = uint32_t(wv); i < uint32_t(RJ) * 16 * NCT; i += NW) {
@@ -607,6 +743,9 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
             float sum = 0.f;
 #pragma unroll
             for (uint32_t k = 0; k < PLANES; ++k) sum += red[k * NRT * TILE + at];
+            if constexpr (G32)
+                if ((tl < 16 ? inf[0] : inf[NCT - 1]) >> (tl % 16) & 1)
+                    sum += non_finite<BITS, META>(p, t, u0 * kUnit, min(u1 * kUnit, p.cols), row0 + rl);
             out[size_t(t) * p.rows + row0 + rl] = sum;
         }
     }
@@ -635,16 +774,17 @@ hipError_t launch_instance(const WideParams &p, hipStream_t stream) {
 
 // Centring costs 5% with two RHS tiles, where unpacking no longer hides under
 // the matrix cores (17408x5120, Q4, 128 RHS: 80.7 us, 76.7 without). Q4 does
-// without it there in group 32, and in group 64 with whole 256-column rows;
-// the other shapes' error was lower before (1.8e-7) and they are centred.
+// without it there in group 64 with whole 256-column rows; the other shapes'
+// error was lower before (1.8e-7) and they are centred. F16 metadata comes in
+// blocks of up to four RHS only, in group 32.
 template <int BITS, int META, bool G32>
 hipError_t launch_tile(const WideParams &p, const WidePlan &pl, hipStream_t stream) {
 #define QMR_WIDE(RT, CT, NW)                                                                                       \
     if (pl.rt == RT && pl.ct == CT && pl.nw == NW) {                                                               \
-        if constexpr (BITS == 4 && CT == 2)                                                                        \
-            if (G32 || (p.group == 64 && p.cols % 256 == 0))                                                       \
-                return launch_instance<BITS, META, G32, false, RT, CT, NW>(p, stream);                             \
-        if constexpr (BITS == 8 || CT == 1 || !G32) return launch_instance<BITS, META, G32, true, RT, CT, NW>(p, stream); \
+        if constexpr (G32 && (META != 2 || CT == 1)) return launch_instance<BITS, META, G32, true, RT, CT, NW>(p, stream); \
+        if constexpr (!G32 && BITS == 4 && CT == 2)                                                                \
+            if (p.group == 64 && p.cols % 256 == 0) return launch_instance<BITS, META, G32, false, RT, CT, NW>(p, stream); \
+        if constexpr (!G32) return launch_instance<BITS, META, G32, true, RT, CT, NW>(p, stream);                  \
     }
     QMR_WIDE(2, 1, 8) QMR_WIDE(4, 1, 4) QMR_WIDE(4, 1, 8) QMR_WIDE(5, 1, 8) QMR_WIDE(8, 1, 8) QMR_WIDE(8, 1, 4)
     QMR_WIDE(4, 2, 4) QMR_WIDE(4, 2, 8) QMR_WIDE(5, 2, 8) QMR_WIDE(7, 2, 4) QMR_WIDE(8, 2, 4)
@@ -659,9 +799,10 @@ struct Regions {
 Regions regions(const AffineArgs &a, const WidePlan &pl) {
     auto up = [](size_t v) { return (v + 255) / 256 * 256; };
     const size_t units = (a.cols + kUnit - 1) / kUnit, ntb = (a.batch + kRhsBlock - 1) / kRhsBlock;
+    const bool g32 = a.group == 32;
     Regions r{};
-    r.expo = up(units * ntb * kImgBytes);
-    r.planes = r.expo + up(size_t(pl.ns) * pl.nw * ntb * kRhsBlock * 4);
+    r.expo = up(units * 2 * ntb * img_bytes(g32));
+    r.planes = r.expo + (g32 ? 0 : up(size_t(pl.ns) * pl.nw * ntb * kRhsBlock * 4));
     r.total = r.planes + (pl.ns > 1 ? size_t(pl.ns) * a.batch * a.rows * 4 : 0);
     return r;
 }
@@ -672,11 +813,12 @@ bool wide_mfma_supported(const AffineArgs &a) {
     if (a.bits != 4 && a.bits != 8) return false;
     if (a.group != 32 && a.group != 64 && a.group != 128) return false;
     if (a.batch < 1 || a.batch > 256 || a.residual || a.up_w) return false;
+    if (a.meta == Meta::F16 && (a.group != 32 || a.batch > 16)) return false;  // no wide block has it
     // 32-bit buffer offsets: codes reach one workgroup's rows past the
     // matrix, images one chunk of units past the row (all read as zeros).
     const uint64_t row_bytes = uint64_t(a.cols) * a.bits / 8;
     const uint64_t ntb = (a.batch + kRhsBlock - 1) / kRhsBlock;
-    const uint64_t img = (uint64_t(a.cols + kUnit - 1) / kUnit + 40) * ntb * kImgBytes;
+    const uint64_t img = (uint64_t(a.cols + kUnit - 1) / kUnit + 40) * 2 * ntb * img_bytes(a.group == 32);
     const uint64_t meta = uint64_t(a.rows) * (a.cols / a.group) * (a.meta == Meta::F32 ? 4 : 2);
     return uint64_t(a.batch) * a.cols * 4 < (1ull << 31) && (uint64_t(a.rows) + 16 * 10) * row_bytes < (1ull << 31) &&
            img < (1ull << 31) && meta < (1ull << 31) && meta >= 32;
@@ -710,6 +852,7 @@ WidePlan plan_wide(const AffineArgs &a, const DeviceLimits &lim, const WidePlan 
     WidePlan best;
     float best_us = 0.f;
     for (const Instance &in : instances) {
+        if (a.meta == Meta::F16 && in.ct != 1) continue;
         if ((force.rt && force.rt != in.rt) || (force.ct && force.ct != in.ct) || (force.nw && force.nw != in.nw)) continue;
         for (const uint32_t ns : {1u, 2u, 3u, 4u, 6u, 8u}) {
             WidePlan pl;
@@ -742,9 +885,9 @@ WideExtent wide_address_extent(uint32_t rows, uint32_t cols, uint32_t n, uint32_
     WideExtent out{};
     const uint32_t units = (cols + kUnit - 1) / kUnit, ntb = (n + kRhsBlock - 1) / kRhsBlock;
     const uint32_t nrb = (rows + 16 * nrt - 1) / (16 * nrt);
-    const WideAddr A{rows, units, ntb, cols / 2};
+    const WideAddr A{rows, units, 2 * ntb, cols / 2, ntb, false};
     out.code_extent = uint64_t(rows) * cols / 2;
-    out.image_extent = uint64_t(units) * ntb * kImgBytes;
+    out.image_extent = uint64_t(units) * 2 * ntb * img_bytes(false);
     auto note = [](uint64_t &mx, uint32_t v, uint32_t so, uint32_t size) {
         if (v != kOut) mx = std::max(mx, uint64_t(v) + so + size);
     };
@@ -758,7 +901,7 @@ WideExtent wide_address_extent(uint32_t rows, uint32_t cols, uint32_t n, uint32_
         for (uint32_t ct = 0; ct < 2 * ntb + 4; ++ct)
             for (uint32_t l = 0; l < 64; ++l) {
                 for (uint32_t f = 0; f < 8; ++f) note(out.image_end, A.frag_v(l, u, ct), A.frag_s(u, ct, f), 16);
-                for (uint32_t sub = 0; sub < 4; ++sub) note(out.image_end, A.sum_at(u, sub, ct, l & 15), 0, 4);
+                for (uint32_t sub = 0; sub < 2; ++sub) note(out.image_end, A.sum_at(u, sub, ct, l & 15), 0, 4);
             }
     }
     return out;
@@ -789,23 +932,26 @@ hipError_t launch_wide_mfma(const AffineArgs &a, const WidePlan &pl, unsigned ch
     p.ups = pl.ups;
     p.w_bytes = uint32_t(uint64_t(a.rows) * a.cols * a.bits / 8);
     p.m_bytes = uint32_t((uint64_t(a.rows) * p.groups * (a.meta == Meta::F32 ? 4 : 2) + 3) / 4 * 4);
-    p.img_bytes = uint32_t(size_t(p.units) * p.ntb * kImgBytes);
-    const uint32_t grid = 2 * p.ntb * pl.ns * pl.nw;
-    if (a.bits == 4)
+    const bool g32 = a.group == 32;
+    p.img_bytes = uint32_t(size_t(p.units) * 2 * p.ntb * img_bytes(g32));
+    const uint32_t tiles = (a.batch + 15) / 16, grid = 2 * p.ntb * pl.ns * pl.nw;
+    const auto prep32 = a.bits == 4 ? wide_prep32_kernel<4> : wide_prep32_kernel<8>;
+    if (g32)
+        hipLaunchKernelGGL(prep32, dim3((p.units * tiles + kPrep32Waves - 1) / kPrep32Waves), dim3(64 * kPrep32Waves), 0,
+                           stream, p, tiles);
+    else if (a.bits == 4)
         hipLaunchKernelGGL(wide_prep_kernel<4>, dim3(grid), dim3(kPrepThreads), 0, stream, p, pl.nw);
     else
         hipLaunchKernelGGL(wide_prep_kernel<8>, dim3(grid), dim3(kPrepThreads), 0, stream, p, pl.nw);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const bool g32 = a.group == 32;
-    if (a.bits == 4)
-        e = a.meta == Meta::F32    ? (g32 ? launch_tile<4, 0, true>(p, pl, stream) : launch_tile<4, 0, false>(p, pl, stream))
-            : a.meta == Meta::BF16 ? (g32 ? launch_tile<4, 1, true>(p, pl, stream) : launch_tile<4, 1, false>(p, pl, stream))
-                                   : (g32 ? launch_tile<4, 2, true>(p, pl, stream) : launch_tile<4, 2, false>(p, pl, stream));
-    else
-        e = a.meta == Meta::F32    ? (g32 ? launch_tile<8, 0, true>(p, pl, stream) : launch_tile<8, 0, false>(p, pl, stream))
-            : a.meta == Meta::BF16 ? (g32 ? launch_tile<8, 1, true>(p, pl, stream) : launch_tile<8, 1, false>(p, pl, stream))
-                                   : (g32 ? launch_tile<8, 2, true>(p, pl, stream) : launch_tile<8, 2, false>(p, pl, stream));
+    auto launch = [&](auto bits) {
+        constexpr int B = decltype(bits)::value;
+        if (a.meta == Meta::F32) return g32 ? launch_tile<B, 0, true>(p, pl, stream) : launch_tile<B, 0, false>(p, pl, stream);
+        if (a.meta == Meta::BF16) return g32 ? launch_tile<B, 1, true>(p, pl, stream) : launch_tile<B, 1, false>(p, pl, stream);
+        return launch_tile<B, 2, true>(p, pl, stream);
+    };
+    e = a.bits == 4 ? launch(std::integral_constant<int, 4>{}) : launch(std::integral_constant<int, 8>{});
     if (e != hipSuccess || pl.ns == 1) return e;
     const uint32_t count = a.batch * a.rows;
     hipLaunchKernelGGL(wide_sum_kernel, dim3(std::min((count + 255) / 256, 2048u)), dim3(256), 0, stream, planes, a.y,

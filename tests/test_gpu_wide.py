@@ -88,3 +88,55 @@ def test_group_32_blocks_on_either_kernel(gpu, rows, cols, bits, batch, wide):
     per = (np.repeat(s, 32) * top + np.repeat(np.abs(b), 32)).reshape(rows, cols)
     bound = 4 * cols * 2.0**-24 * (np.abs(x).astype(np.float64) @ per.T.astype(np.float64))
     assert (np.abs(got[0] - got[1]) <= bound).all()
+
+# A wide block whose columns fill units, quarters and two RHS tiles, blocks of
+# three and four over the lines that send them to the wide kernel, and the
+# three metadata types.
+@pytest.mark.parametrize("name,rows,cols,bits,batch", [("matmul_affine_wide", 65, 1056, 4, 33),
+                                                       ("matmul_affine_wide_bf16", 40, 4128, 8, 7),
+                                                       ("matmul_affine_bf16", 33, 9248, 4, 4),
+                                                       ("matmul_affine_f16meta", 33, 12320, 8, 3)])
+def test_group_32_keeps_every_bit_of_x(gpu, name, rows, cols, bits, batch):
+    """x as the vector-ALU kernel multiplies it: FP32 values of any size. A
+    token's columns spread over 2^60, one is 2^118 where the weights are zero,
+    and then one is Inf and one NaN."""
+    rng = np.random.default_rng(rows + cols)
+    meta = {"wide": "f32", "bf16": "bf16", "f16meta": "f16"}[name.split("_")[-1]]
+    store = {"f32": lambda v: v, "bf16": synth.f32_to_bf16_bits, "f16": lambda v: v.astype(np.float16).view(np.uint16)}[meta]
+    load = {"f32": lambda v: v, "bf16": synth.bf16_bits_to_f32, "f16": synth.f16_bits_to_f32}[meta]
+    middle = 2 ** (bits - 1)
+    codes = rng.integers(0, 2**bits, (rows, cols), dtype=np.uint32)
+    s = store(rng.uniform(0.002, 0.02, (rows, cols // 32)).astype(np.float32))
+    b = store(rng.uniform(0.001, 0.01, (rows, cols // 32)).astype(np.float32))
+    x = (rng.standard_normal((batch, cols)) * np.exp2(rng.integers(-40, 21, (batch, cols)))).astype(np.float32)
+    big = cols - 5
+    codes[:, big], x[:, big] = middle, np.float32(2.0**118)
+    b[:, big // 32] = store(-middle * load(s)[:, big // 32])
+    codes[:, 37] |= 1
+    pack = 32 // bits
+    w = (codes.reshape(rows, -1, pack) << (np.arange(pack, dtype=np.uint32) * bits)).sum(axis=2, dtype=np.uint32)
+    want = oracle.matmul_f64(w.ravel(), s.ravel(), b.ravel(), meta, x, rows, cols, bits, 32, batch, THREADS).reshape(batch, rows)
+    # A group's three products, its scaling and its bias are each rounded to
+    # 2^-24 of the sum of magnitudes at the very most, and 32 more join
+    # classes and splits.
+    weight = np.repeat(load(s), 32, axis=1) * np.abs(codes.astype(np.float64) - middle) + \
+        np.repeat(np.abs(load(b).astype(np.float64) + middle * load(s)), 32, axis=1)
+    bound = 1.01 * (cols / 32 * 5 + 32) * 2.0**-24 * (np.abs(x).astype(np.float64) @ weight.T)
+    params = [rows, cols, bits, 32, batch]
+    buffers = [*upload_matrix(gpu, w, s, b), gpu.upload_f32(x.ravel()), gpu.alloc_f32(batch * rows)]
+    gpu.dispatch(name, buffers, params)
+    assert gpu.last_hip_kernel() == "wide_mfma_kernel"
+    assert (np.abs(gpu.read_f32(buffers[4], batch * rows).reshape(batch, rows) - want) <= bound).all()
+    x[1, 37], x[2, 40] = np.inf, np.nan
+    buffers[3] = gpu.upload_f32(x.ravel())
+    got = []
+    try:
+        for plan in ((0, 0), (-1, 0)):
+            gpu.set_gemv_plan(*plan)
+            gpu.dispatch(name, buffers, params)
+            got.append(gpu.read_f32(buffers[4], batch * rows).reshape(batch, rows))
+    finally:
+        gpu.set_gemv_plan(0, 0)
+    assert np.isposinf(got[0][1]).all() and np.isnan(got[0][2]).all() and np.isfinite(np.delete(got[0], (1, 2), axis=0)).all()
+    for kind in (np.isnan, np.isposinf, np.isneginf):
+        assert np.array_equal(kind(got[0]), kind(got[1]))
