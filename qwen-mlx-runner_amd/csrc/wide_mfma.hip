@@ -813,6 +813,9 @@ bool wide_mfma_supported(const AffineArgs &a) {
     if (a.bits != 4 && a.bits != 8) return false;
     if (a.group != 32 && a.group != 64 && a.group != 128) return false;
     if (a.batch < 1 || a.batch > 256 || a.residual || a.up_w) return false;
+    // Codes at any 4-byte offset can be loaded, but such views run on the
+    // vector ALU as blocks, in FP32, which group 32 alone keeps here.
+    if (a.group != 32 && reinterpret_cast<uintptr_t>(a.w) % 16 != 0) return false;
     if (a.meta == Meta::F16 && (a.group != 32 || a.batch > 16)) return false;  // no wide block has it
     // 32-bit buffer offsets: codes reach one workgroup's rows past the
     // matrix, images one chunk of units past the row (all read as zeros).

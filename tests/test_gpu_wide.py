@@ -8,7 +8,7 @@ import pytest
 
 import oracle
 import qmr.synth as synth
-from helpers import upload_matrix
+from helpers import assert_gate, upload_matrix
 
 pytestmark = pytest.mark.gpu
 THREADS = min(16, os.cpu_count() or 1)
@@ -140,3 +140,28 @@ def test_group_32_keeps_every_bit_of_x(gpu, name, rows, cols, bits, batch):
     assert np.isposinf(got[0][1]).all() and np.isnan(got[0][2]).all() and np.isfinite(np.delete(got[0], (1, 2), axis=0)).all()
     for kind in (np.isnan, np.isposinf, np.isneginf):
         assert np.array_equal(kind(got[0]), kind(got[1]))
+
+
+@pytest.mark.parametrize("rows,cols,bits,group,meta,batch", [(65, 1056, 4, 32, "f32", 18), (40, 1056, 8, 32, "bf16", 5),
+                                                             (65, 1088, 4, 64, "bf16", 18), (40, 1152, 8, 128, "f32", 6)])
+@pytest.mark.parametrize("static", [False, True])
+def test_wide_views_at_four_byte_offsets(gpu, rows, cols, bits, group, meta, batch, static):
+    """Codes that are not 16-byte aligned keep FP32 products: group 32 on the
+    wide kernel, the others as blocks on the vector ALU."""
+    rng = np.random.default_rng(rows + cols)
+    top = 2**bits
+    w = rng.integers(0, 2**32, rows * cols * bits // 32, dtype=np.uint32)
+    sf = rng.uniform(0.002, 0.02, rows * cols // group).astype(np.float32)
+    bf = (-top / 2 * sf + rng.normal(0, 1e-3, sf.size)).astype(np.float32)
+    s, b = (synth.f32_to_bf16_bits(sf), synth.f32_to_bf16_bits(bf)) if meta == "bf16" else (sf, bf)
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    want = oracle.matmul_f64(w, s, b, meta, x, rows, cols, bits, group, batch, THREADS)
+    pad = lambda a: np.concatenate([np.full(4, 0xA5, np.uint8), np.ascontiguousarray(a).view(np.uint8).ravel()])
+    buffers = [gpu.upload_bytes(pad(a)) for a in (w, s, b, x, np.zeros(batch * rows + 4, np.float32))]
+    name, params = "matmul_affine_wide" + NAME[meta], [rows, cols, bits, group, batch]
+    command = gpu.begin()
+    command.encode(name, buffers, params, rows * 32, 64, [4] * 5, static_scratch=static)
+    command.finish()
+    assert gpu.last_hip_kernel() == ("wide_mfma_kernel" if group == 32 else "affine_gemv_kernel")
+    assert_gate(gpu.read_f32(buffers[4], batch * rows, 4), want)
+    assert not gpu.read_f32(buffers[4], 4, 4 + 4 * batch * rows).any()
