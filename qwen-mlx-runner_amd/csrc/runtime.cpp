@@ -153,6 +153,10 @@ int guarded(F &&f) {
         if (!(ok)) fail(__VA_ARGS__); \
     } while (0)
 
+// Device buffers end with a whole word: the wide kernel loads 16-bit metadata a
+// word at a time, also where a view has an odd number of elements.
+size_t whole_words(size_t bytes) { return bytes < 4 ? 4 : (bytes + 3) / 4 * 4; }
+
 void check_hip(hipError_t e, const char *what) {
     if (e != hipSuccess) throw Error{QMR_ERR_DEVICE, std::string(what) + ": " + hipGetErrorString(e)};
 }
@@ -289,7 +293,7 @@ int upload_staged_views(::qmr_device *device, const StagedView *views, size_t n,
                 if (d) hipFree(d);
         };
         hipError_t e = hipSuccess;
-        for (size_t i = 0; i < n && e == hipSuccess; ++i) e = hipMalloc(&dst[i], views[i].bytes > 0 ? views[i].bytes : 4);
+        for (size_t i = 0; i < n && e == hipSuccess; ++i) e = hipMalloc(&dst[i], whole_words(views[i].bytes));
         if (e != hipSuccess) {
             free_all();
             check_hip(e, "hipMalloc");
@@ -927,7 +931,7 @@ int qmr_buffer_alloc(qmr_device *device, size_t bytes, qmr_buffer **out) {
                                            std::to_string(device->max_alloc));
         check_hip(hipSetDevice(device->ordinal), "hipSetDevice");
         void *p = nullptr;
-        check_hip(hipMalloc(&p, n), "hipMalloc");
+        check_hip(hipMalloc(&p, whole_words(n)), "hipMalloc");
         // Zeroed on the device stream and waited for, so the fill is ordered
         // before both later launches and host reads.
         hipError_t e = hipMemsetAsync(p, 0, n, device->stream);
@@ -956,7 +960,7 @@ int qmr_buffer_upload(qmr_device *device, const void *data, size_t bytes, qmr_bu
                                                std::to_string(device->max_alloc));
         check_hip(hipSetDevice(device->ordinal), "hipSetDevice");
         void *p = nullptr;
-        check_hip(hipMalloc(&p, bytes), "hipMalloc");
+        check_hip(hipMalloc(&p, whole_words(bytes)), "hipMalloc");
         hipError_t e = hipMemcpy(p, data, bytes, hipMemcpyHostToDevice);
         if (e != hipSuccess) {
             hipFree(p);
