@@ -300,14 +300,16 @@ const char *qmr_last_hip_kernel(const qmr_device *device);
 /* LDS bytes one workgroup may allocate on this device. */
 size_t qmr_device_max_lds(const qmr_device *device);
 /* Host-only check of the wide block kernel's addressing (no device needed):
- * walks every code, x-fragment and group-sum load its contraction launch
- * issues for rows x cols (a multiple of 256) times batch RHS with row_tiles
- * (8 or 17) 16-row tiles per workgroup, and writes out[0] = the largest end
- * (byte offset + size) of the in-range code loads, out[1] = the code view's
- * size, out[2] = the largest end of the in-range image loads, out[3] = the
- * image workspace's size. Loads outside a view take the vector offset past
- * every view and read zeros. */
-int qmr_wide_address_extent(uint32_t rows, uint32_t cols, uint32_t batch, uint32_t row_tiles, uint64_t *out);
+ * walks every code, image and metadata load its contraction launch issues,
+ * through the functions that the kernel takes its offsets from. params: rows,
+ * cols, bits, group, batch; f32_metadata: 1, or 0 for 16-bit metadata; plan:
+ * 16-row tiles, 16-RHS tiles, waves per workgroup (a compiled instance's) and
+ * K splits. Writes, for the codes, the images and the metadata, the largest
+ * end (byte offset + size) of the in-range loads and the view's size (of
+ * 16-bit metadata up to the end of its last word), out[0..5], and out[6] = 1
+ * if a metadata load missed an element that it is for. Loads outside a view
+ * take the vector offset past every view and read zeros. */
+int qmr_wide_address_extent(const uint32_t *params, int f32_metadata, const uint32_t *plan, uint64_t *out);
 
 #ifdef __cplusplus
 }

@@ -240,14 +240,15 @@ bool wide_mfma_supported(const AffineArgs &a);
 WidePlan plan_wide(const AffineArgs &a, const DeviceLimits &lim, const WidePlan &force = WidePlan{});
 size_t wide_mfma_workspace(const AffineArgs &a, const WidePlan &pl);
 hipError_t launch_wide_mfma(const AffineArgs &a, const WidePlan &pl, unsigned char *workspace, hipStream_t stream);
-// Host-side walk of every code, x-fragment and group-sum load the wide
-// contraction kernel issues for a shape with nrt row tiles per block: the
-// largest end (offset + size) of the in-range loads in the code view and in
-// the image workspace, beside the two extents.
+bool wide_instance(const WidePlan &pl);  // rt, ct and nw are a compiled instance's
+// Host-side walk of every code, image and metadata load the wide contraction
+// kernel issues under a plan (its ns: the splits asked for): the largest end
+// (offset + size) of the in-range loads in each view, beside the views'
+// extents, and whether a metadata load missed an element that it is for.
 struct WideExtent {
-    uint64_t code_end, code_extent, image_end, image_extent;
+    uint64_t code_end, code_extent, image_end, image_extent, meta_end, meta_extent, meta_short;
 };
-WideExtent wide_address_extent(uint32_t rows, uint32_t cols, uint32_t n, uint32_t nrt);
+WideExtent wide_address_extent(const AffineArgs &a, WidePlan pl);
 
 // The plan the GEMV launcher would use (for tests and tuning reports).
 GemvPlan plan_affine_gemv(const AffineArgs &a, GemvPlan forced, const DeviceLimits &lim);

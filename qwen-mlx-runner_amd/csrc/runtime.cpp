@@ -1411,17 +1411,27 @@ static int encode_command(qmr_command *command, const char *cname, qmr_buffer *c
     });
 }
 
-int qmr_wide_address_extent(uint32_t rows, uint32_t cols, uint32_t batch, uint32_t row_tiles, uint64_t *out) {
+int qmr_wide_address_extent(const uint32_t *params, int f32_metadata, const uint32_t *plan, uint64_t *out) {
     return guarded([&]() -> int {
-        ensure(out != nullptr, "qmr_wide_address_extent: null output");
-        ensure(rows > 0 && cols > 0 && cols % 256 == 0 && batch >= 1 && batch <= 256 &&
-                   (row_tiles == 8 || row_tiles == 17) && uint64_t(rows) * cols / 2 < (1ull << 31),
-               "qmr_wide_address_extent: unsupported shape");
-        const qmr::WideExtent e = qmr::wide_address_extent(rows, cols, batch, row_tiles);
-        out[0] = e.code_end;
-        out[1] = e.code_extent;
-        out[2] = e.image_end;
-        out[3] = e.image_extent;
+        ensure(params != nullptr && plan != nullptr && out != nullptr, "qmr_wide_address_extent: null argument");
+        qmr::AffineArgs a{};
+        a.rows = params[0];
+        a.cols = params[1];
+        a.bits = params[2];
+        a.group = params[3];
+        a.batch = params[4];
+        a.meta = f32_metadata ? qmr::Meta::F32 : qmr::Meta::BF16;
+        qmr::WidePlan pl;
+        pl.rt = plan[0];
+        pl.ct = plan[1];
+        pl.nw = plan[2];
+        pl.ns = plan[3];
+        ensure(a.rows > 0 && a.cols > 0 && a.group > 0 && a.cols % a.group == 0 && qmr::wide_mfma_supported(a) &&
+                   qmr::wide_instance(pl) && pl.ns >= 1 && pl.ns <= 99,
+               "qmr_wide_address_extent: unsupported shape or plan");
+        const qmr::WideExtent e = qmr::wide_address_extent(a, pl);
+        const uint64_t all[] = {e.code_end, e.code_extent, e.image_end, e.image_extent, e.meta_end, e.meta_extent, e.meta_short};
+        std::copy(std::begin(all), std::end(all), out);
         return QMR_OK;
     });
 }

@@ -143,24 +143,30 @@ constexpr size_t wide_lds_bytes(int nrt, int nct, int nw) {
     return std::max(2 * meta_bytes(nrt, nw) + nw * code_bytes(nrt), red + kFlagBytes);
 }
 
-// Byte offsets of the contraction kernel's code, x-fragment and group-sum
-// loads, as the per-lane vector offset and the wave-uniform scalar offset of
-// a buffer load. A load outside its view (a row past the matrix, columns past
-// the row, a unit past the split, an RHS tile past the images) gets the vector
-// offset kOut, which by itself lies past every view's extent, so it reads
-// zeros whether or not the range check adds the scalar offset (kOut plus any
-// scalar offset here stays below 2^32); every other load has voffset +
-// soffset + size within its view. qmr_wide_address_extent walks these on the
-// host.
+// Byte offsets of the contraction kernel's loads, as the per-lane vector
+// offset and the wave-uniform scalar offset of a buffer load. A load outside
+// its view (a row past the matrix, columns past the row, a unit past the
+// split, an RHS tile past the images) gets the vector offset kOut, which by
+// itself lies past every view's extent, so it reads zeros whether or not the
+// range check adds the scalar offset (kOut plus any scalar offset here stays
+// below 2^32); every other load has voffset + soffset + size within its view.
+// The kernel takes every offset from these functions, and
+// qmr_wide_address_extent walks them on the host.
 struct WideAddr {
-    uint32_t rows, units, tiles, row_bytes;  // tiles: RHS tiles with an image
+    uint32_t rows, units, tiles, row_bytes;  // units: end of the split's; tiles: RHS tiles with an image
     uint32_t ntb;                            // pairs of RHS tiles
     bool g32;
-    // Lane (row16, piece) loads 16 bytes of row row0 + 16 rt + row16 at byte
-    // 64 seg + 16 piece (a unit is one 64-byte segment of Q4, two of Q8).
-    __host__ __device__ uint32_t code_v(uint32_t row0, uint32_t rt, uint32_t row16, uint32_t piece, uint32_t seg) const {
-        return row0 + 16 * rt + row16 < rows && 64 * seg + 16 * piece < row_bytes ? (row0 + row16) * row_bytes + 16 * piece
-                                                                                 : kOut;
+    // Lane (row16, piece) loads 16 bytes of rows row + 16 rt (row = the row
+    // block's first plus row16) at byte 64 seg + 16 piece; a unit is one
+    // 64-byte segment of Q4, two of Q8. Tiles from code_tiles on have no such
+    // row, or the row no such bytes.
+    __host__ __device__ uint32_t row_tiles(uint32_t row) const { return row < rows ? (rows - row + 15) / 16 : 0; }
+    __host__ __device__ uint32_t code_tiles(uint32_t row_tiles, uint32_t u, uint32_t seg, uint32_t piece) const {
+        return u < units && 64 * seg + 16 * piece < row_bytes ? row_tiles : 0;
+    }
+    __host__ __device__ uint32_t code_at(uint32_t row, uint32_t piece) const { return row * row_bytes + 16 * piece; }
+    __host__ __device__ uint32_t code_v(uint32_t rt, uint32_t code_tiles, uint32_t code_at) const {
+        return rt < code_tiles ? code_at : kOut;
     }
     __host__ __device__ uint32_t code_s(uint32_t rt, uint32_t seg) const { return rt * 16 * row_bytes + 64 * seg; }
     // Fragment f of RHS tile ct in unit u; lane l reads 16 bytes.
@@ -177,6 +183,36 @@ struct WideAddr {
         return u < units && ct < tiles ? image(u, ct) + img_sums(g32) + sub * 64 + r16 * 4 : kOut;
     }
 };
+
+// The scales or biases of eight consecutive groups from group g of a row on:
+// 16 bytes of a window of whole words and its rest 16 bytes further. The window
+// begins in the word of the first one, or as far before it as the view's end
+// asks; skip() elements of it are not wanted. A view of 16-bit elements ends
+// in a whole word (no buffer is shorter), whose other half is not used.
+template <int META>
+struct MetaWindow {
+    static constexpr uint32_t kSize = META == 0 ? 4 : 2;    // bytes of an element
+    static constexpr uint32_t kWords = META == 0 ? 8 : 5;
+    uint32_t groups, bytes;  // of a row; of the view
+    __host__ __device__ uint32_t at(uint32_t row, uint32_t g) const { return (row * groups + g) * kSize; }
+    __host__ __device__ uint32_t window(uint32_t at) const {
+        const uint32_t word = at & ~3u, last = bytes - 4 * kWords;
+        return word < last ? word : last;
+    }
+    __host__ __device__ uint32_t skip(uint32_t at) const { return (at - window(at)) / kSize; }
+};
+
+// Metadata item i of thread tid: the row within the block and the groups
+// 8 j.. of a chunk.
+__host__ __device__ constexpr uint32_t units_per_chunk(bool g32) { return g32 ? 1 : 2; }  // four slots each
+struct MetaItem {
+    uint32_t row, j;
+};
+__host__ __device__ inline MetaItem meta_item(uint32_t tid, uint32_t i, uint32_t threads, uint32_t items_per_row) {
+    const uint32_t k = tid + i * threads;  // items per row: a power of two
+    return MetaItem{k >> (31 - __builtin_clz(items_per_row)), tid & (items_per_row - 1)};
+}
+__host__ __device__ constexpr uint32_t items_per_thread(uint32_t nrt) { return (nrt + 7) / 8; }
 
 struct WideParams {
     const uint32_t *w;
@@ -365,11 +401,10 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
     constexpr int KG = G32 ? 1 : 2;       // K steps per group (or half of 128)
     constexpr int PARTS = parts_of(G32);  // of x
     constexpr int SL = 4 / KG;            // slots (groups or halves of 128) per unit
-    constexpr uint32_t UPC = 4 / SL;      // units per chunk: four slots, one bias product
+    constexpr uint32_t UPC = units_per_chunk(G32);
     constexpr int THREADS = 64 * NW_, PITCH = meta_pitch(NW_);
-    constexpr int PER_T = (NRT + 7) / 8;  // metadata items per thread and chunk
+    constexpr int PER_T = items_per_thread(NRT);  // metadata items per thread and chunk
     constexpr int RJ = (ROWS + 63) / 64;  // waves' worth of rows
-    constexpr uint32_t BSZ = META == 0 ? 4 : 2;
     extern __shared__ __align__(16) unsigned char lds[];
     const int tid = threadIdx.x;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);  // the wave's K class (uniform)
@@ -385,7 +420,7 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
     const uint32_t rb = pair % p.nrb, split = pair / p.nrb;
     const uint32_t row0 = rb * ROWS, ct0 = cb * NCT;
     const uint32_t u0 = split * p.ups, u1 = min(u0 + p.ups, p.units);
-    const WideAddr A{p.rows, u1, G32 ? (p.n + 15) / 16 : 2 * p.ntb, p.cols / (32 / BITS) * 4, p.ntb, G32};
+    const WideAddr A{p.rows, u1, (p.n + 15) / 16, p.cols / (32 / BITS) * 4, p.ntb, G32};
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint32_t *>(p.w), 0, int(p.w_bytes), kRsrcWord3);
     const __amdgpu_buffer_rsrc_t ir = __builtin_amdgcn_make_buffer_rsrc(p.img, 0, int(p.img_bytes), kRsrcWord3);
@@ -395,16 +430,14 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
 
     // ---- codes: lane (row16, piece) loads 16 bytes of a row of every tile.
     const uint32_t row16 = uint32_t(lane) >> 2, piece = uint32_t(lane) & 3;
-    const uint32_t code_base = (row0 + row16) * A.row_bytes + 16 * piece;
-    const uint32_t tiles_in = row0 + row16 < p.rows ? (p.rows - row0 - row16 + 15) / 16 : 0;  // tiles with a row in the matrix
+    const uint32_t code_at = A.code_at(row0 + row16, piece), row_tiles = A.row_tiles(row0 + row16);
     u4 raw[SEG][NRT];
     auto load_codes = [&](u4 (&dst)[NRT], uint32_t u, int sg) {
-        const uint32_t seg = u * SEG + uint32_t(sg);
-        const uint32_t tiles = u < u1 && 64 * seg + 16 * piece < A.row_bytes ? tiles_in : 0u;
+        const uint32_t seg = u * SEG + uint32_t(sg), tiles = A.code_tiles(row_tiles, u, seg, piece);
 #pragma unroll
         for (int rt = 0; rt < NRT; ++rt)
             dst[rt] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                 wr, int(uint32_t(rt) < tiles ? code_base : kOut), int(A.code_s(uint32_t(rt), seg)), 0));
+                                                 wr, int(A.code_v(uint32_t(rt), tiles, code_at)), int(A.code_s(uint32_t(rt), seg)), 0));
     };
     auto put_codes = [&](const u4 (&src)[NRT]) {
 #pragma unroll
@@ -412,23 +445,20 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
             *reinterpret_cast<u4 *>(turn + (rt * 16 + row16) * kCodePitch + piece * 16) = src[rt];
     };
     // ---- metadata of chunk c (units u0 + UPC*NW*c ..): item (row, j) = eight
-    // consecutive groups of one row. A window of whole words that holds them
-    // and lies inside the view is loaded; the groups are shifted into place
-    // when they are used.
+    // consecutive groups of one row, shifted into place when they are used.
     const uint32_t gpu = kUnit / p.group;      // groups per unit
     const uint32_t gpc = gpu * UPC * NW;       // groups per chunk: 4 NW (group 128: 2 NW)
     const uint32_t ipr = gpc / 8;              // items per row
-    const uint32_t ish = 31u - __builtin_clz(ipr);
-    const uint32_t mj = uint32_t(tid) & (ipr - 1);
+    const MetaWindow<META> M{p.groups, p.m_bytes};
+    const uint32_t mj = meta_item(uint32_t(tid), 0, THREADS, ipr).j;
     const uint32_t g_first = gpu * u0, g_end = min(p.groups, gpu * u1);
-    constexpr uint32_t WIN = META == 0 ? 8 : 5;  // words of a window
+    constexpr uint32_t WIN = MetaWindow<META>::kWords;
     struct MStage {
         u4 s0[PER_T], b0[PER_T];
         std::conditional_t<META == 0, u4, uint32_t> s1[PER_T], b1[PER_T];
     };
-    auto item_row = [&](int i) { return (uint32_t(tid) + uint32_t(i) * THREADS) >> ish; };
-    auto item_at = [&](uint32_t rl, uint32_t c) { return ((row0 + rl) * p.groups + g_first + c * gpc + 8 * mj) * BSZ; };
-    auto window = [&](uint32_t at) { return min(at & ~3u, p.m_bytes - 4 * WIN); };
+    auto item_row = [&](int i) { return meta_item(uint32_t(tid), uint32_t(i), THREADS, ipr).row; };
+    auto item_at = [&](uint32_t rl, uint32_t c) { return M.at(row0 + rl, g_first + c * gpc + 8 * mj); };
     auto item_live = [&](uint32_t rl, uint32_t c) {
         return rl < uint32_t(ROWS) && row0 + rl < p.rows && g_first + c * gpc + 8 * mj < g_end;
     };
@@ -436,7 +466,7 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
 #pragma unroll
         for (int i = 0; i < PER_T; ++i) {
             const uint32_t rl = item_row(i);
-            const uint32_t at = item_live(rl, c) ? window(item_at(rl, c)) : kOut;
+            const uint32_t at = item_live(rl, c) ? M.window(item_at(rl, c)) : kOut;
             st.s0[i] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(sr, int(at), 0, 0));
             st.b0[i] = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(br, int(at), 0, 0));
             if constexpr (META == 0) {
@@ -483,7 +513,7 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
 #pragma unroll
         for (int i = 0; i < PER_T; ++i) {
             const uint32_t rl = item_row(i);
-            const uint32_t at = item_at(rl, c), skip = item_live(rl, c) ? (at - window(at)) / BSZ : 0u;
+            const uint32_t skip = item_live(rl, c) ? M.skip(item_at(rl, c)) : 0u;
             float sv[8], bv[8];
             eight(sv, st.s0[i], st.s1[i], skip);
             eight(bv, st.b0[i], st.b1[i], skip);
@@ -807,6 +837,13 @@ Regions regions(const AffineArgs &a, const WidePlan &pl) {
     return r;
 }
 
+// Whole rounds of a workgroup's waves per split; splits left without a unit go.
+WidePlan split_units(WidePlan pl, uint32_t units) {
+    pl.ups = ((units + pl.ns - 1) / pl.ns + pl.nw - 1) / pl.nw * pl.nw;
+    pl.ns = (units + pl.ups - 1) / pl.ups;
+    return pl;
+}
+
 }  // namespace
 
 bool wide_mfma_supported(const AffineArgs &a) {
@@ -827,17 +864,20 @@ bool wide_mfma_supported(const AffineArgs &a) {
            img < (1ull << 31) && meta < (1ull << 31) && meta >= 32;
 }
 
+namespace {
+struct Instance {
+    uint32_t rt, ct, nw, per_cu;  // per_cu: workgroups that fit a CU (LDS, registers)
+};
+constexpr Instance kInstances[] = {{2, 1, 8, 1}, {4, 1, 4, 3}, {4, 1, 8, 1}, {5, 1, 8, 1}, {8, 1, 8, 1}, {8, 1, 4, 2},
+                                   {4, 2, 4, 2}, {4, 2, 8, 1}, {5, 2, 8, 1}, {7, 2, 4, 2}, {8, 2, 4, 2}};
+}  // namespace
+
 // The plan is the cheapest of the compiled instances and up to eight K splits
 // under a model of what a workgroup does, fitted to 1500 timings (17 shapes
 // from 1024x1024 to 17408x5120, 4 to 256 RHS, both code sizes, groups 32, 64
 // and 128; its choice is on average 2.6% slower than the fastest plan, and
 // what is furthest off, 1.4x, are 200 RHS over 900 rows).
 WidePlan plan_wide(const AffineArgs &a, const DeviceLimits &lim, const WidePlan &force) {
-    struct Instance {
-        uint32_t rt, ct, nw, per_cu;  // per_cu: workgroups that fit a CU (LDS, registers)
-    };
-    constexpr Instance instances[] = {{2, 1, 8, 1}, {4, 1, 4, 3}, {4, 1, 8, 1}, {5, 1, 8, 1}, {8, 1, 8, 1}, {8, 1, 4, 2},
-                                      {4, 2, 4, 2}, {4, 2, 8, 1}, {5, 2, 8, 1}, {7, 2, 4, 2}, {8, 2, 4, 2}};
     // Microseconds: a call, a group's products per row tile (one or two RHS
     // tiles), the rest of a group step, a metadata chunk, the factor of a CU
     // with less than two waves per SIMD, a round of workgroups, the sum launch
@@ -847,14 +887,9 @@ WidePlan plan_wide(const AffineArgs &a, const DeviceLimits &lim, const WidePlan 
     const uint32_t units = (a.cols + kUnit - 1) / kUnit, nct = (a.batch + 15) / 16;
     const uint32_t steps = a.group == 32 ? 4 : 2;  // group steps per unit
     const uint32_t cus = uint32_t(std::max(lim.num_cus, 1));
-    auto split = [&](WidePlan pl) {
-        pl.ups = ((units + pl.ns - 1) / pl.ns + pl.nw - 1) / pl.nw * pl.nw;
-        pl.ns = (units + pl.ups - 1) / pl.ups;
-        return pl;
-    };
     WidePlan best;
     float best_us = 0.f;
-    for (const Instance &in : instances) {
+    for (const Instance &in : kInstances) {
         if (a.meta == Meta::F16 && in.ct != 1) continue;
         if ((force.rt && force.rt != in.rt) || (force.ct && force.ct != in.ct) || (force.nw && force.nw != in.nw)) continue;
         for (const uint32_t ns : {1u, 2u, 3u, 4u, 6u, 8u}) {
@@ -863,7 +898,7 @@ WidePlan plan_wide(const AffineArgs &a, const DeviceLimits &lim, const WidePlan 
             pl.ct = in.ct;
             pl.nw = in.nw;
             pl.ns = force.ns ? force.ns : ns;
-            pl = split(pl);
+            pl = split_units(pl, units);
             // A split's classes all have a unit; its planes fit the scratch of
             // the encode that allocates nothing, so that both take one plan.
             if (!force.ns && ns > 1 && (units / ns < in.nw || regions(a, pl).total > QMR_STATIC_SCRATCH_BYTES)) continue;
@@ -884,30 +919,75 @@ WidePlan plan_wide(const AffineArgs &a, const DeviceLimits &lim, const WidePlan 
 
 size_t wide_mfma_workspace(const AffineArgs &a, const WidePlan &pl) { return regions(a, pl).total; }
 
-WideExtent wide_address_extent(uint32_t rows, uint32_t cols, uint32_t n, uint32_t nrt) {
+WideExtent wide_address_extent(const AffineArgs &a, WidePlan pl) {
     WideExtent out{};
-    const uint32_t units = (cols + kUnit - 1) / kUnit, ntb = (n + kRhsBlock - 1) / kRhsBlock;
-    const uint32_t nrb = (rows + 16 * nrt - 1) / (16 * nrt);
-    const WideAddr A{rows, units, 2 * ntb, cols / 2, ntb, false};
-    out.code_extent = uint64_t(rows) * cols / 2;
-    out.image_extent = uint64_t(units) * 2 * ntb * img_bytes(false);
+    const bool g32 = a.group == 32;
+    const uint32_t units = (a.cols + kUnit - 1) / kUnit, ntb = (a.batch + kRhsBlock - 1) / kRhsBlock;
+    const uint32_t groups = a.cols / a.group, gpu = kUnit / a.group;
+    const uint32_t nrb = (a.rows + 16 * pl.rt - 1) / (16 * pl.rt), ncb = ((a.batch + 15) / 16 + pl.ct - 1) / pl.ct;
+    const uint32_t segs = a.bits / 4;
+    pl = split_units(pl, units);
+    const uint64_t meta_view = uint64_t(a.rows) * groups * (a.meta == Meta::F32 ? 4 : 2);
+    out.code_extent = uint64_t(a.rows) * a.cols * a.bits / 8;
+    out.image_extent = uint64_t(units) * 2 * ntb * img_bytes(g32);
+    out.meta_extent = (meta_view + 3) / 4 * 4;
     auto note = [](uint64_t &mx, uint32_t v, uint32_t so, uint32_t size) {
-        if (v != kOut) mx = std::max(mx, uint64_t(v) + so + size);
+        if (v < kOut) mx = std::max(mx, uint64_t(v) + so + size);
     };
-    // Every unit, and those past the row that the prefetches reach.
-    for (uint32_t u = 0; u < units + 32; ++u) {
-        for (uint32_t rb = 0; rb < nrb; ++rb)
-            for (uint32_t rt = 0; rt < nrt; ++rt)
+    auto meta_loads = [&](auto window, uint32_t row0, uint32_t g_first, uint32_t g_end, uint32_t c) {
+        constexpr uint32_t rest = 4 * decltype(window)::kWords - 16;
+        const uint32_t threads = 64 * pl.nw, gpc = gpu * units_per_chunk(g32) * pl.nw;
+        for (uint32_t tid = 0; tid < threads; ++tid)
+            for (uint32_t i = 0; i < items_per_thread(pl.rt); ++i) {
+                const MetaItem m = meta_item(tid, i, threads, gpc / 8);
+                const uint32_t g = g_first + c * gpc + 8 * m.j, row = row0 + m.row;
+                if (m.row >= 16 * pl.rt || row >= a.rows || g >= g_end) continue;
+                const uint32_t at = window.at(row, g), first = window.window(at);
+                note(out.meta_end, first, 0, 16);
+                note(out.meta_end, first, 16, rest);
+                // What is used of them: the eight groups up to the split's end.
+                const uint32_t wanted = std::min(8u, g_end - g) * window.kSize;
+                out.meta_short = std::max<uint64_t>(out.meta_short, first + window.skip(at) * window.kSize != at ||
+                                                                        at + wanted > first + 16 + rest);
+            }
+    };
+    for (uint32_t split = 0; split < pl.ns; ++split) {
+        const uint32_t u0 = split * pl.ups, u1 = std::min(u0 + pl.ups, units);
+        const WideAddr A{a.rows, u1, (a.batch + 15) / 16, a.cols / (32 / a.bits) * 4, ntb, g32};
+        // Every unit, and those past the split that the prefetches reach.
+        for (uint32_t u = u0; u < u1 + 2 * pl.nw; ++u) {
+            for (uint32_t row0 = 0; row0 < nrb * 16 * pl.rt; row0 += 16 * pl.rt)
                 for (uint32_t l = 0; l < 64; ++l)
-                    note(out.code_end, A.code_v(rb * 16 * nrt, rt, l >> 2, l & 3, u), A.code_s(rt, u), 16);
-        // RHS tiles up to a block of four past the images.
-        for (uint32_t ct = 0; ct < 2 * ntb + 4; ++ct)
-            for (uint32_t l = 0; l < 64; ++l) {
-                for (uint32_t f = 0; f < 8; ++f) note(out.image_end, A.frag_v(l, u, ct), A.frag_s(u, ct, f), 16);
-                for (uint32_t sub = 0; sub < 2; ++sub) note(out.image_end, A.sum_at(u, sub, ct, l & 15), 0, 4);
+                    for (uint32_t seg = u * segs; seg < (u + 1) * segs; ++seg) {
+                        const uint32_t row = row0 + (l >> 2), tiles = A.code_tiles(A.row_tiles(row), u, seg, l & 3);
+                        for (uint32_t rt = 0; rt < pl.rt; ++rt)
+                            note(out.code_end, A.code_v(rt, tiles, A.code_at(row, l & 3)), A.code_s(rt, seg), 16);
+                    }
+            for (uint32_t ct = 0; ct < ncb * pl.ct; ++ct)
+                for (uint32_t l = 0; l < 64; ++l) {
+                    for (uint32_t f = 0; f < 4 * parts_of(g32); ++f)
+                        note(out.image_end, A.frag_v(l, u, ct), A.frag_s(u, ct, f), 16);
+                    for (uint32_t sub = 0; sub < (g32 ? 4u : 2u); ++sub)
+                        note(out.image_end, A.sum_at(u, sub, ct, l & 15), 0, 4);
+                }
+        }
+        const uint32_t per = units_per_chunk(g32) * pl.nw, chunks = (u1 - u0 + per - 1) / per;
+        for (uint32_t c = 0; c <= chunks; ++c)
+            for (uint32_t row0 = 0; row0 < nrb * 16 * pl.rt; row0 += 16 * pl.rt) {
+                const uint32_t g_first = gpu * u0, g_end = std::min(groups, gpu * u1);
+                if (a.meta == Meta::F32)
+                    meta_loads(MetaWindow<0>{groups, uint32_t(out.meta_extent)}, row0, g_first, g_end, c);
+                else
+                    meta_loads(MetaWindow<1>{groups, uint32_t(out.meta_extent)}, row0, g_first, g_end, c);
             }
     }
     return out;
+}
+
+bool wide_instance(const WidePlan &pl) {
+    for (const Instance &in : kInstances)
+        if (in.rt == pl.rt && in.ct == pl.ct && in.nw == pl.nw) return true;
+    return false;
 }
 
 hipError_t launch_wide_mfma(const AffineArgs &a, const WidePlan &pl, unsigned char *workspace, hipStream_t stream) {

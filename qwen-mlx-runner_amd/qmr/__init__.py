@@ -138,7 +138,7 @@ def lib() -> C.CDLL:
         "qmr_buffer_release": (None, [vp]),
         "qmr_command_begin": (C.c_int, [vp, C.POINTER(vp)]),
         "qmr_encode": (C.c_int, [vp, C.c_char_p, C.POINTER(vp), szp, sz, u32p, sz, sz, sz]),
-        "qmr_wide_address_extent": (C.c_int, [C.c_uint32, C.c_uint32, C.c_uint32, C.c_uint32, C.POINTER(C.c_uint64)]),
+        "qmr_wide_address_extent": (C.c_int, [C.POINTER(C.c_uint32), C.c_int, C.POINTER(C.c_uint32), C.POINTER(C.c_uint64)]),
         "qmr_encode_static": (C.c_int, [vp, C.c_char_p, C.POINTER(vp), szp, sz, u32p, sz, sz, sz]),
         "qmr_command_mark": (C.c_int, [vp, C.POINTER(C.c_int)]),
         "qmr_command_delay": (C.c_int, [vp, C.c_uint32]),
@@ -197,12 +197,12 @@ def _s(v: Optional[str]) -> Optional[bytes]:
 
 # ---- host-only contract (no GPU needed) ----
 
-def wide_address_extent(rows: int, cols: int, batch: int, row_tiles: int) -> tuple[int, int, int, int]:
-    """qmr_wide_address_extent: (largest end of the wide kernel's in-range code
-    loads, code view bytes, largest end of its in-range image loads, image
-    workspace bytes), walked on the host."""
-    out = (C.c_uint64 * 4)()
-    _check(lib().qmr_wide_address_extent(rows, cols, batch, row_tiles, out))
+def wide_address_extent(params: Sequence[int], f32_metadata: bool, plan: Sequence[int]) -> tuple[int, ...]:
+    """qmr_wide_address_extent: for the wide kernel's codes, images and
+    metadata the largest end of its in-range loads and the view's bytes, then
+    whether a metadata load missed an element, walked on the host."""
+    out = (C.c_uint64 * 7)()
+    _check(lib().qmr_wide_address_extent(_u32(params), int(f32_metadata), _u32(plan), out))
     return tuple(int(v) for v in out)
 
 

@@ -246,16 +246,40 @@ def test_pack_bf16_exact_patterns_and_supported_formats():
         assert not qmr.supported_bf16_quantization(bits, group)
 
 
-@pytest.mark.parametrize("rows,cols,batch", [(17408, 5120, 128), (17408, 5120, 256), (5120, 17408, 64),
-                                             (16 * 17 * 3 + 5, 512, 33), (9, 256, 1), (300, 1024, 200)])
-@pytest.mark.parametrize("row_tiles", [8, 17])
-def test_wide_kernel_loads_stay_inside_their_views(rows, cols, batch, row_tiles):
-    """Every code, x-fragment and group-sum load of the wide contraction
-    kernel (walked on the host through the kernel's own offset functions):
-    loads outside a view go through the vector offset past every view, and
-    the in-range ones end inside theirs. The last code byte and the last
-    image byte are reached, so the walk covers the views to their ends."""
-    code_end, code_extent, image_end, image_extent = qmr.wide_address_extent(rows, cols, batch, row_tiles)
-    assert code_end == code_extent == rows * cols // 2
-    assert image_extent == (cols // 64) * ((batch + 31) // 32) * 8448
-    assert image_end <= image_extent and image_end > image_extent - 8448
+# Whole and ragged rows; a last unit of 32, 64 and 128 columns; odd counts of
+# 16-bit scales per row and in all; the smallest view; RHS in one tile, past a
+# tile and in all sixteen.
+WIDE_SHAPES = [(2048, 5120, 4, 64, 128), (16 * 17 * 3 + 5, 512, 4, 64, 33), (9, 256, 4, 64, 1), (300, 1088, 4, 64, 200),
+               (129, 1056, 4, 32, 17), (65, 864, 8, 32, 256), (33, 1984, 8, 64, 31), (81, 1408, 4, 128, 16),
+               (17, 640, 8, 128, 34), (16, 64, 4, 64, 5), (15, 160, 8, 32, 8), (257, 4224, 8, 128, 70)]
+WIDE_PLANS = [(2, 1, 8), (4, 1, 4), (4, 1, 8), (5, 1, 8), (8, 1, 8), (8, 1, 4), (4, 2, 4), (4, 2, 8), (5, 2, 8), (7, 2, 4),
+              (8, 2, 4)]
+
+
+@pytest.mark.parametrize("rows,cols,bits,group,batch", WIDE_SHAPES)
+@pytest.mark.parametrize("f32", [False, True])
+def test_wide_kernel_loads_stay_inside_their_views(rows, cols, bits, group, batch, f32):
+    """Every code, image and metadata load of the wide contraction kernel
+    (walked on the host through the functions the kernel takes its offsets
+    from): loads outside a view go through the vector offset past every view,
+    and the in-range ones end inside theirs. The last bytes of the codes, the
+    metadata and the last image are reached, so the walk covers the views to
+    their ends, and no metadata load misses what it is for."""
+    units, tiles = -(-cols // 128), -(-batch // 16)
+    meta = rows * (cols // group) * (4 if f32 else 2)
+    image = {32: 12544}.get(group, 8448)
+    for plan in WIDE_PLANS:
+        for splits in (1, 2, 5):
+            code_end, code, image_end, images, meta_end, meta_extent, short = \
+                qmr.wide_address_extent([rows, cols, bits, group, batch], f32, [*plan, splits])
+            assert code_end == code == rows * cols * bits // 8
+            assert images == units * (tiles + tiles % 2) * image
+            assert image_end <= images and image_end > images - (1 + tiles % 2) * image
+            assert meta_extent == (meta + 3) // 4 * 4 and meta_end == meta_extent and short == 0
+
+
+def test_wide_kernel_walk_refuses_what_the_kernel_does_not_take():
+    for params, plan in (([9, 256, 4, 64, 1], [17, 2, 4, 1]), ([9, 256, 4, 64, 1], [8, 2, 4, 0]),
+                         ([9, 250, 4, 64, 1], [8, 2, 4, 1]), ([1, 64, 4, 64, 5], [8, 2, 4, 1]),
+                         ([9, 256, 4, 64, 257], [8, 2, 4, 1]), ([9, 256, 3, 64, 1], [8, 2, 4, 1])):
+        err(qmr.wide_address_extent, params, True, plan)
