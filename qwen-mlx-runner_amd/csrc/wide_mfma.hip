@@ -50,7 +50,6 @@ using namespace mfma;
 
 typedef uint32_t u2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u3 __attribute__((ext_vector_type(3)));
-typedef int i4 __attribute__((ext_vector_type(4)));
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 
 // Codes as f16: Q4 as subnormals (the code times 2^-20), Q8 as 1024 + code;
@@ -116,15 +115,17 @@ __device__ __forceinline__ f4 product(const u4 &x, const u4 &codes, const f4 &c)
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, x), __builtin_bit_cast(h8, codes), c, 0, 0, 0);
 }
 
-constexpr int kPrepThreads = 1024;
 constexpr uint32_t kUnit = 128;                 // columns per unit: four K steps of the MFMA
 constexpr int kRhsBlock = 32;                   // RHS tiles come in pairs
 constexpr int kFragBytes = 1024;                // one MFMA A fragment (64 lanes x 16 B)
 // An image: one unit of one RHS tile. Its fragments [K step][part], then the
-// column sums [quarter (group 32) or half][16] f32.
+// column sums [quarter (group 32) or half][16] f32, then (not group 32) the
+// factors [half][16] that undo the power of two of x and of the codes, as the
+// exponent byte of an FP32 value.
 constexpr uint32_t parts_of(bool g32) { return g32 ? 3 : 2; }
 constexpr uint32_t img_sums(bool g32) { return 4 * parts_of(g32) * kFragBytes; }
 constexpr uint32_t img_bytes(bool g32) { return img_sums(g32) + 256; }
+constexpr uint32_t kImgFactors = img_sums(false) + 128;
 
 // A wave's piece of LDS: codes on their way to operand order (64 bytes of each
 // row, one unit of Q4 or half a unit of Q8; rows 80 bytes apart so that
@@ -182,6 +183,10 @@ struct WideAddr {
     __host__ __device__ uint32_t sum_at(uint32_t u, uint32_t sub, uint32_t ct, uint32_t r16) const {
         return u < units && ct < tiles ? image(u, ct) + img_sums(g32) + sub * 64 + r16 * 4 : kOut;
     }
+    // Factors of RHS 16 ct + 4 q .. + 3 over half `sub`: four bytes.
+    __host__ __device__ uint32_t factor_at(uint32_t u, uint32_t sub, uint32_t ct, uint32_t q) const {
+        return u < units && ct < tiles ? image(u, ct) + kImgFactors + sub * 16 + q * 4 : kOut;
+    }
 };
 
 // The scales or biases of eight consecutive groups from group g of a row on:
@@ -221,7 +226,6 @@ struct WideParams {
     const float *x;
     float *y;              // output, or the first K split's plane
     unsigned char *img;    // [units][2 ntb] images
-    int *expo;             // [ns * nw][32 ntb] exponents e of the images' 2^-e (not group 32)
     uint32_t rows, cols, n;       // n = RHS count
     uint32_t group;
     uint32_t units, groups;       // 128-column units (the last may be partial) and quant groups per row
@@ -231,114 +235,15 @@ struct WideParams {
     uint32_t w_bytes, m_bytes, img_bytes;  // extents of the views
 };
 
-// ---- 1. Activation images: one workgroup per (RHS tile, K class), every wave
-// one unit at a time, lane (t16, c4) the columns 8*c4.. of the four K steps of
-// RHS t16. The scale 2^-e is shared by an RHS's units of one class, so that
-// the contraction can accumulate over them. ----
-template <int BITS>
-__global__ __launch_bounds__(kPrepThreads) void wide_prep_kernel(WideParams p, uint32_t nw) {
-    constexpr uint32_t kWavesP = kPrepThreads / 64;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    __shared__ uint32_t red[kWavesP][16];
-    const uint32_t ct = blockIdx.x % (2 * p.ntb), cls = blockIdx.x / (2 * p.ntb);
-    const uint32_t split = cls / nw, w = cls % nw;
-    const uint32_t u0 = split * p.ups, u1 = min(u0 + p.ups, p.units);
-    const uint32_t t16 = uint32_t(lane) & 15, c4 = uint32_t(lane) >> 4;
-    const uint32_t t = ct * 16 + t16;
-    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float *>(p.x), 0, int(p.n * p.cols * 4u), kRsrcWord3);
-    const uint32_t first = u0 + w + uint32_t(wave) * nw, step = kWavesP * nw;
-    auto load = [&](float (&xv)[4][8], uint32_t u) {
-#pragma unroll
-        for (uint32_t ks = 0; ks < 4; ++ks)
-            load_x8(xv[ks], xr, t, u * kUnit + 32 * ks + 8 * c4, p.cols, t < p.n && u < u1);
-    };
-    uint32_t mb = 0;
-    auto largest = [&](const float (&xv)[4][8]) {
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-            for (int j = 0; j < 8; ++j) mb = max(mb, __float_as_uint(xv[ks][j]) & 0x7FFFFFFFu);
-    };
-    float x0[4][8];
-    load(x0, first);
-    largest(x0);
-    for (uint32_t u = first + step; u < u1; u += step) {
-        float xv[4][8];
-        load(xv, u);
-        largest(xv);
-    }
-    mb = max(mb, uint32_t(__shfl_xor(int(mb), 16)));
-    mb = max(mb, uint32_t(__shfl_xor(int(mb), 32)));
-    if (lane < 16) red[wave][lane] = mb;
-    __syncthreads();
-    mb = red[0][t16];
-#pragma unroll
-    for (uint32_t v = 1; v < kWavesP; ++v) mb = max(mb, red[v][t16]);
-    int e = 0;
-    if (mb != 0u && mb < 0x7F800000u) {
-        e = int(mb >> 23) - 127 - 14;  // max * 2^-e in [2^14, 2^15) for normal max
-        e = e < -100 ? -100 : (e > 100 ? 100 : e);
-    }
-    const float sc = __uint_as_float(uint32_t(127 - e) << 23);
-    if (tid < 16) p.expo[size_t(cls) * (kRhsBlock * p.ntb) + t] = e;
-    auto store = [&](const float (&xv)[4][8], uint32_t u) {
-        unsigned char *img = p.img + (size_t(u) * 2 * p.ntb + ct) * img_bytes(false);
-        unsigned char *frag = img + lane * 16;
-        float quarter[4];  // this lane's part of the sum of each K step's 32 columns
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            const float(&v)[8] = xv[ks];
-            quarter[ks] = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
-            u4 hw, lw;
-#pragma unroll
-            for (int e2 = 0; e2 < 4; ++e2) {
-                const float v0 = v[k_of<BITS>(2 * e2)], v1 = v[k_of<BITS>(2 * e2 + 1)];
-                hw[e2] = hi_pair(v0, v1, sc);
-                lw[e2] = lo_pair(v0, v1, sc, hw[e2]);
-            }
-            *reinterpret_cast<u4 *>(frag + 2 * ks * kFragBytes) = hw;
-            *reinterpret_cast<u4 *>(frag + (2 * ks + 1) * kFragBytes) = lw;
-        }
-        // Sums of the unit's halves, with the codes' power of two, so that b *
-        // S adds to s * D.
-        const float cs = sc * (1.f / float(1u << kWideExp<BITS>));
-        float *S = reinterpret_cast<float *>(img + img_sums(false)) + t16;
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            quarter[ks] += __shfl_xor(quarter[ks], 16);
-            quarter[ks] += __shfl_xor(quarter[ks], 32);
-        }
-        if (c4 == 0) {
-            S[0] = (quarter[0] + quarter[1]) * cs;
-            S[16] = (quarter[2] + quarter[3]) * cs;
-        }
-    };
-    if (first < u1) store(x0, first);
-    for (uint32_t u = first + step; u < u1; u += step) {
-        float xv[4][8];
-        load(xv, u);
-        store(xv, u);
-    }
-}
+// ---- 1. Activation images: a wave per unit and RHS tile, lane (t16, c4) the
+// columns 8*c4.. of the four K steps of RHS t16. ----
+constexpr uint32_t kPrepWaves = 4;
 
-// The images of group 32: a wave per unit and RHS tile, lane (t16, c4) as
-// above. Parts are cut off, not rounded: three times eight bits are all of a
-// value's, and the first does not overflow. Inf and NaN stay out of the
+// Group 32: parts are cut off, not rounded: three times eight bits are all of
+// a value's, and the first does not overflow. Inf and NaN stay out of the
 // fragments; NaN in place of their quarter's sum says that there are some.
-constexpr uint32_t kPrep32Waves = 4;
 template <int BITS>
-__global__ __launch_bounds__(64 * kPrep32Waves) void wide_prep32_kernel(WideParams p, uint32_t tiles) {
-    const uint32_t i = blockIdx.x * kPrep32Waves + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const uint32_t u = i / tiles, ct = i % tiles;
-    if (u >= p.units) return;
-    const uint32_t t16 = lane & 15, c4 = lane >> 4, t = ct * 16 + t16;
-    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float *>(p.x), 0, int(p.n * p.cols * 4u), kRsrcWord3);
-    unsigned char *img = p.img + (size_t(u) * 2 * p.ntb + ct) * img_bytes(true);
-    float xv[4][8];
-#pragma unroll
-    for (uint32_t ks = 0; ks < 4; ++ks) load_x8(xv[ks], xr, t, u * kUnit + 32 * ks + 8 * c4, p.cols, t < p.n);
+__device__ __forceinline__ void put_image32(float (&xv)[4][8], unsigned char *img, uint32_t lane) {
 #pragma unroll
     for (uint32_t ks = 0; ks < 4; ++ks) {
         float(&v)[8] = xv[ks];
@@ -352,7 +257,7 @@ __global__ __launch_bounds__(64 * kPrep32Waves) void wide_prep32_kernel(WidePara
         float sum = bad + (((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7])));
         sum += __shfl_xor(sum, 16);
         sum += __shfl_xor(sum, 32);
-        if (c4 == 0) reinterpret_cast<float *>(img + img_sums(true))[ks * 16 + t16] = sum;
+        if (lane < 16) reinterpret_cast<float *>(img + img_sums(true))[ks * 16 + lane] = sum;
         u4 part[3];
 #pragma unroll
         for (int e2 = 0; e2 < 4; ++e2) {
@@ -368,6 +273,71 @@ __global__ __launch_bounds__(64 * kPrep32Waves) void wide_prep32_kernel(WidePara
 #pragma unroll
         for (int k = 0; k < 3; ++k) *reinterpret_cast<u4 *>(img + (3 * ks + k) * kFragBytes + lane * 16) = part[k];
     }
+}
+
+// The other groups: hi and lo f16 halves under a power of two of its own for
+// every RHS and 64 columns, as the block kernels have it for every group: a
+// column loses bits only where another of the same 64 is 2^17 times larger.
+// (One per RHS and K class: 4e-5 off beside one column of 1e8.)
+template <int BITS>
+__device__ __forceinline__ void put_image64(const float (&xv)[4][8], unsigned char *img, uint32_t lane) {
+#pragma unroll
+    for (uint32_t half = 0; half < 2; ++half) {
+        uint32_t mb = 0;
+        float sum = 0.f;
+#pragma unroll
+        for (uint32_t ks = 2 * half; ks < 2 * half + 2; ++ks) {
+            const float(&v)[8] = xv[ks];
+            sum += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+#pragma unroll
+            for (int j = 0; j < 8; ++j) mb = max(mb, __float_as_uint(v[j]) & 0x7FFFFFFFu);
+        }
+        sum += __shfl_xor(sum, 16);
+        sum += __shfl_xor(sum, 32);
+        mb = max(mb, uint32_t(__shfl_xor(int(mb), 16)));
+        mb = max(mb, uint32_t(__shfl_xor(int(mb), 32)));
+        int e = 0;
+        if (mb != 0u && mb < 0x7F800000u) {
+            e = int(mb >> 23) - 127 - 14;  // max * 2^-e in [2^14, 2^15) for normal max
+            e = e < -100 ? -100 : (e > 100 ? 100 : e);
+        }
+        if (lane < 16) {
+            reinterpret_cast<float *>(img + img_sums(false))[half * 16 + lane] = sum;
+            img[kImgFactors + half * 16 + lane] = static_cast<unsigned char>(127 + e + kWideExp<BITS>);
+        }
+        const float sc = __uint_as_float(uint32_t(127 - e) << 23);
+#pragma unroll
+        for (uint32_t ks = 2 * half; ks < 2 * half + 2; ++ks) {
+            u4 hw, lw;
+#pragma unroll
+            for (int e2 = 0; e2 < 4; ++e2) {
+                const float v0 = xv[ks][k_of<BITS>(2 * e2)], v1 = xv[ks][k_of<BITS>(2 * e2 + 1)];
+                hw[e2] = hi_pair(v0, v1, sc);
+                lw[e2] = lo_pair(v0, v1, sc, hw[e2]);
+            }
+            *reinterpret_cast<u4 *>(img + 2 * ks * kFragBytes + lane * 16) = hw;
+            *reinterpret_cast<u4 *>(img + (2 * ks + 1) * kFragBytes + lane * 16) = lw;
+        }
+    }
+}
+
+template <int BITS, bool G32>
+__global__ __launch_bounds__(64 * kPrepWaves) void wide_prep_kernel(WideParams p, uint32_t tiles) {
+    const uint32_t i = blockIdx.x * kPrepWaves + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const uint32_t u = i / tiles, ct = i % tiles;
+    if (u >= p.units) return;
+    const uint32_t t = ct * 16 + (lane & 15);
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>(p.x), 0, int(p.n * p.cols * 4u), kRsrcWord3);
+    float xv[4][8];
+#pragma unroll
+    for (uint32_t ks = 0; ks < 4; ++ks)
+        load_x8(xv[ks], xr, t, u * kUnit + 32 * ks + 8 * (lane >> 4), p.cols, t < p.n);
+    unsigned char *img = p.img + (size_t(u) * 2 * p.ntb + ct) * img_bytes(G32);
+    if constexpr (G32)
+        put_image32<BITS>(xv, img, lane);
+    else
+        put_image64<BITS>(xv, img, lane);
 }
 
 // What Inf and NaN among the columns [c0, c1) of an RHS add to row r of a
@@ -572,6 +542,15 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
                 ir, int(A.sum_at(u, G32 ? uint32_t(q) : uint32_t(q) & 1, ct0 + uint32_t(ct), uint32_t(r16))), 0, 0));
     };
 
+    // Factors of a unit's half for the lane's four RHS: exponent bytes.
+    uint32_t fe[2][NCT];
+    auto load_factors = [&](uint32_t (&dst)[NCT], uint32_t u, uint32_t half) {
+        if constexpr (!G32)
+#pragma unroll
+            for (int ct = 0; ct < NCT; ++ct)
+                dst[ct] = __builtin_amdgcn_raw_buffer_load_b32(ir, int(A.factor_at(u, half, ct0 + uint32_t(ct), uint32_t(q))), 0, 0);
+    };
+
     f4 acc[NRT][NCT];
     float sa[NCT];
     bool bad[NCT] = {};  // group 32: Inf or NaN in the columns of sa
@@ -591,6 +570,7 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
         for (int sg = 0; sg < SEG; ++sg) load_codes(raw[sg], u, sg);
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) load_x(xf[ks], u, uint32_t(ks));
+        for (uint32_t half = 0; half < 2; ++half) load_factors(fe[half], u, half);
         load_s(sa, 0);
         __builtin_amdgcn_sched_barrier(0);  // every request before any use
         put_meta(st, 0);
@@ -650,12 +630,20 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
                         }
                     };
                     f4 d[2][NCT];
+                    f4 fac[NCT];
+                    if constexpr (!G32)
+#pragma unroll
+                        for (int ct = 0; ct < NCT; ++ct)
+#pragma unroll
+                            for (int v = 0; v < 4; ++v)
+                                fac[ct][v] = __uint_as_float((v < 3 ? fe[sl & 1][ct] << (23 - 8 * v) : fe[sl & 1][ct] >> 1) & 0x7F800000u);
                     auto close = [&](int rt) {
 #pragma unroll
                         for (int ct = 0; ct < NCT; ++ct)
 #pragma unroll
                             for (int v = 0; v < 4; ++v)
-                                acc[rt][ct][v] = __builtin_fmaf(sv[rt % 3], d[rt & 1][ct][v], acc[rt][ct][v]);
+                                acc[rt][ct][v] = __builtin_fmaf(sv[rt % 3], G32 ? d[rt & 1][ct][v] : d[rt & 1][ct][v] * fac[ct][v],
+                                                                acc[rt][ct][v]);
                     };
                     fetch(0);
                     if (NRT > 1) fetch(1);
@@ -681,6 +669,7 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                     for (int k = 0; k < KG; ++k) load_x(xf[ks + k], un, uint32_t(ks + k));
+                    load_factors(fe[sl & 1], un, uint32_t(sl & 1));
                     close(NRT - 1);
                 }
                 wave_lds_sync();
@@ -706,26 +695,12 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
         lds_barrier();
     }
 
-    // ---- the classes meet in LDS, each wave's sums times 2^(e + code
-    // exponent), and are added in order. A wave stores 64 rows of an RHS at a
-    // time.
+    // ---- the classes meet in LDS and are added in order. A wave stores 64
+    // rows of an RHS at a time.
     lds_barrier();  // every wave is done with its piece
     float *red = reinterpret_cast<float *>(lds);
     constexpr int TILE = NCT * 256 + kRedPad;
     constexpr uint32_t PLANES = NW > 4 ? 4 : NW;
-    if constexpr (!G32) {
-#pragma unroll
-        for (int ct = 0; ct < NCT; ++ct) {
-            const uint32_t t = (ct0 + uint32_t(ct)) * 16 + uint32_t(q) * 4;
-            i4 e{0, 0, 0, 0};
-            if (ct0 + uint32_t(ct) < 2 * p.ntb)
-                e = *reinterpret_cast<const i4 *>(p.expo + size_t(split * NW + uint32_t(wv)) * (kRhsBlock * p.ntb) + t);
-#pragma unroll
-            for (int rt = 0; rt < NRT; ++rt)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) acc[rt][ct][v] = ldexpf(acc[rt][ct][v], e[v] + kWideExp<BITS>);
-        }
-    }
     auto place = [&](int rt, int ct, int v) -> float & {
         return red[((wv % int(PLANES)) * NRT + rt) * TILE + (ct * 4 + v) * 64 + lane];
     };
@@ -824,15 +799,14 @@ hipError_t launch_tile(const WideParams &p, const WidePlan &pl, hipStream_t stre
 
 // Regions of the workspace.
 struct Regions {
-    size_t expo, planes, total;
+    size_t planes, total;
 };
 Regions regions(const AffineArgs &a, const WidePlan &pl) {
     auto up = [](size_t v) { return (v + 255) / 256 * 256; };
     const size_t units = (a.cols + kUnit - 1) / kUnit, ntb = (a.batch + kRhsBlock - 1) / kRhsBlock;
     const bool g32 = a.group == 32;
     Regions r{};
-    r.expo = up(units * 2 * ntb * img_bytes(g32));
-    r.planes = r.expo + (g32 ? 0 : up(size_t(pl.ns) * pl.nw * ntb * kRhsBlock * 4));
+    r.planes = up(units * 2 * ntb * img_bytes(g32));
     r.total = r.planes + (pl.ns > 1 ? size_t(pl.ns) * a.batch * a.rows * 4 : 0);
     return r;
 }
@@ -969,6 +943,8 @@ WideExtent wide_address_extent(const AffineArgs &a, WidePlan pl) {
                         note(out.image_end, A.frag_v(l, u, ct), A.frag_s(u, ct, f), 16);
                     for (uint32_t sub = 0; sub < (g32 ? 4u : 2u); ++sub)
                         note(out.image_end, A.sum_at(u, sub, ct, l & 15), 0, 4);
+                    for (uint32_t sub = 0; sub < 2 && !g32; ++sub)
+                        note(out.image_end, A.factor_at(u, sub, ct, l >> 4), 0, 4);
                 }
         }
         const uint32_t per = units_per_chunk(g32) * pl.nw, chunks = (u1 - u0 + per - 1) / per;
@@ -998,7 +974,6 @@ hipError_t launch_wide_mfma(const AffineArgs &a, const WidePlan &pl, unsigned ch
     p.b = a.b;
     p.x = a.x;
     p.img = workspace;
-    p.expo = reinterpret_cast<int *>(workspace + r.expo);
     float *planes = reinterpret_cast<float *>(workspace + r.planes);
     p.y = pl.ns > 1 ? planes : a.y;
     p.plane = pl.ns > 1 ? a.batch * a.rows : 0;
@@ -1017,15 +992,10 @@ hipError_t launch_wide_mfma(const AffineArgs &a, const WidePlan &pl, unsigned ch
     p.m_bytes = uint32_t((uint64_t(a.rows) * p.groups * (a.meta == Meta::F32 ? 4 : 2) + 3) / 4 * 4);
     const bool g32 = a.group == 32;
     p.img_bytes = uint32_t(size_t(p.units) * 2 * p.ntb * img_bytes(g32));
-    const uint32_t tiles = (a.batch + 15) / 16, grid = 2 * p.ntb * pl.ns * pl.nw;
-    const auto prep32 = a.bits == 4 ? wide_prep32_kernel<4> : wide_prep32_kernel<8>;
-    if (g32)
-        hipLaunchKernelGGL(prep32, dim3((p.units * tiles + kPrep32Waves - 1) / kPrep32Waves), dim3(64 * kPrep32Waves), 0,
-                           stream, p, tiles);
-    else if (a.bits == 4)
-        hipLaunchKernelGGL(wide_prep_kernel<4>, dim3(grid), dim3(kPrepThreads), 0, stream, p, pl.nw);
-    else
-        hipLaunchKernelGGL(wide_prep_kernel<8>, dim3(grid), dim3(kPrepThreads), 0, stream, p, pl.nw);
+    const uint32_t tiles = (a.batch + 15) / 16;
+    const auto prep = a.bits == 4 ? (g32 ? wide_prep_kernel<4, true> : wide_prep_kernel<4, false>)
+                                  : (g32 ? wide_prep_kernel<8, true> : wide_prep_kernel<8, false>);
+    hipLaunchKernelGGL(prep, dim3((p.units * tiles + kPrepWaves - 1) / kPrepWaves), dim3(64 * kPrepWaves), 0, stream, p, tiles);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     auto launch = [&](auto bits) {
