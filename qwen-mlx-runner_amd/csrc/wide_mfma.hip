@@ -3,9 +3,9 @@
 // computed in the factored form
 //     y[t][r] = sum_g ( s[r,g] * D[r,t,g] + b[r,g] * S[t,g] ),
 //     D[r,t,g] = sum_{c in g} q[r,c] * x[t,c],  S[t,g] = sum_{c in g} x[t,c].
-// D runs on v_mfma_f32_16x16x32_f16 with exact integer codes (f16 subnormals,
-// as in mfma_common.hpp, or centred ones) against x split into hi/lo f16 parts, so it is
-// accurate to about 2^-22, or, in group 32, on v_mfma_f32_16x16x32_bf16 against
+// D runs on v_mfma_f32_16x16x32_f16 with exact centred codes against x split
+// into hi/lo f16 parts, accurate to 2^-22 of the value and 2^-40 of the largest
+// of its RHS and 64 columns, or, in group 32, on v_mfma_f32_16x16x32_bf16 against
 // the three bf16 parts of x, which are all of it; the scales multiply D in FP32 and the bias term is
 // an FP32 matrix product of S and b (v_mfma_f32_16x16x4_f32 over four groups
 // at a time).
@@ -49,31 +49,33 @@ namespace {
 using namespace mfma;
 
 typedef uint32_t u2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u3 __attribute__((ext_vector_type(3)));
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 
-// Codes as f16: Q4 as subnormals (the code times 2^-20), Q8 as 1024 + code;
-// centred, less the middle of their range (8 or 128), which goes into the
-// group's bias as middle * scale. Uncentred, s * D and b * S are large and
-// cancel: at 5120 columns 2.4e-7 against 64 bits for Q4 and 2.6e-7 for Q8,
-// centred 1.4e-7 and 1.2e-7. (Q4 as 1024 + code: 1.3e-7, but 10% slower with
-// two RHS tiles; without the shifts, from subnormals of 2^-24, the matrix
-// cores' sums are off by 6e-6.)
-template <int BITS>
-constexpr int kWideExp = BITS == 4 ? 20 : 0;
+// Codes as f16, centred: less the middle of their range (8 or 128), which goes
+// into the group's bias as middle * scale. Uncentred, s * D and b * S are large
+// and cancel: at 5120 columns 2.4e-7 against 64 bits for Q4 and 2.6e-7 for Q8.
+// A code in the low bits of 1024 (in bits 4-7 of 64) is that number plus the
+// code; less the middle too it is exact, and a normal number: as subnormals of
+// 2^-20 (Q4) the sums lose bits beside large columns.
 constexpr float middle_of(int bits) { return bits == 4 ? 8.f : 128.f; }
-template <int BITS, bool CENTRED>
-__device__ __forceinline__ h8 wide_unpack(const u2 &w) {
+// Masks and numbers stay in registers, so that one v_and_or_b32 does both.
+template <int BITS>
+struct CodeConsts {
+    uint32_t low = BITS == 4 ? 0x000F000Fu : 0x00FF00FFu, high = 0x00F000F0u;
+    uint32_t at_low = 0x64006400u, at_high = 0x54005400u;
+    __device__ __forceinline__ CodeConsts() { asm("" : "+s"(low), "+s"(high), "+v"(at_low), "+v"(at_high)); }
+};
+template <int BITS>
+__device__ __forceinline__ u4 f16_codes(const u2 &w, const CodeConsts<BITS> &c) {
+    const u2 up = w >> 8;
+    const _Float16 k = _Float16(1024 + middle_of(BITS)), m = _Float16(64 + 8);
+    auto low = [&](uint32_t v) { return (v & c.low) | c.at_low; };
+    auto high = [&](uint32_t v) { return (v & c.high) | c.at_high; };
     if constexpr (BITS == 4) {
-        const u4 c[1] = {u4{w.x, 0u, 0u, 0u}};
-        const h8 v = unpack<4>(c, 0);
-        return CENTRED ? v - __builtin_bit_cast(_Float16, uint16_t(0x0080)) : v;  // 8 * 2^-20
+        const h8 v = __builtin_bit_cast(h8, u4{low(w.x), high(w.x), low(up.x), high(up.x)});
+        return __builtin_bit_cast(u4, v - h8{k, k, m, m, k, k, m, m});
     } else {
-        static_assert(CENTRED, "1024 + code");
-        const h8 v = __builtin_bit_cast(
-            h8, u4{(w.x & 0x00FF00FFu) | 0x64006400u, ((w.x >> 8) & 0x00FF00FFu) | 0x64006400u,
-                   (w.y & 0x00FF00FFu) | 0x64006400u, ((w.y >> 8) & 0x00FF00FFu) | 0x64006400u});
-        return v - _Float16(1152);
+        return __builtin_bit_cast(u4, __builtin_bit_cast(h8, u4{low(w.x), low(up.x), low(w.y), low(up.y)}) - k);
     }
 }
 
@@ -120,8 +122,8 @@ constexpr int kRhsBlock = 32;                   // RHS tiles come in pairs
 constexpr int kFragBytes = 1024;                // one MFMA A fragment (64 lanes x 16 B)
 // An image: one unit of one RHS tile. Its fragments [K step][part], then the
 // column sums [quarter (group 32) or half][16] f32, then (not group 32) the
-// factors [half][16] that undo the power of two of x and of the codes, as the
-// exponent byte of an FP32 value.
+// factors [half][16] that undo the power of two of x, as the exponent byte of an
+// FP32 value.
 constexpr uint32_t parts_of(bool g32) { return g32 ? 3 : 2; }
 constexpr uint32_t img_sums(bool g32) { return 4 * parts_of(g32) * kFragBytes; }
 constexpr uint32_t img_bytes(bool g32) { return img_sums(g32) + 256; }
@@ -303,7 +305,7 @@ __device__ __forceinline__ void put_image64(const float (&xv)[4][8], unsigned ch
         }
         if (lane < 16) {
             reinterpret_cast<float *>(img + img_sums(false))[half * 16 + lane] = sum;
-            img[kImgFactors + half * 16 + lane] = static_cast<unsigned char>(127 + e + kWideExp<BITS>);
+            img[kImgFactors + half * 16 + lane] = static_cast<unsigned char>(127 + e);
         }
         const float sc = __uint_as_float(uint32_t(127 - e) << 23);
 #pragma unroll
@@ -362,7 +364,7 @@ __device__ float non_finite(const WideParams &p, uint32_t t, uint32_t c0, uint32
 
 // ---- 2. The contraction. Lane (r16, q) of a wave: row r16 of every row
 // tile, K chunk q of every K step; D element v of a tile is RHS 4q + v. ----
-template <int BITS, int META, bool G32, bool CENTRED, int NRT, int NCT, int NW_>
+template <int BITS, int META, bool G32, int NRT, int NCT, int NW_>
 __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
     constexpr uint32_t NW = NW_;
     constexpr int ROWS = 16 * NRT;
@@ -397,6 +399,7 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
     const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p.s), 0, int(p.m_bytes), kRsrcWord3);
     const __amdgpu_buffer_rsrc_t br = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p.b), 0, int(p.m_bytes), kRsrcWord3);
     const f4 zero{0.f, 0.f, 0.f, 0.f};
+    const CodeConsts<BITS> consts;
 
     // ---- codes: lane (row16, piece) loads 16 bytes of a row of every tile.
     const uint32_t row16 = uint32_t(lane) >> 2, piece = uint32_t(lane) & 3;
@@ -491,7 +494,7 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
 #pragma unroll
             for (uint32_t k = 0; k < 8; ++k) {  // past the split's groups there may be a neighbour's
                 sv[k] = g + k < g_end ? sv[k] : 0.f;
-                bv[k] = g + k < g_end ? CENTRED ? __builtin_fmaf(middle_of(BITS), sv[k], bv[k]) : bv[k] : 0.f;
+                bv[k] = g + k < g_end ? __builtin_fmaf(middle_of(BITS), sv[k], bv[k]) : 0.f;
                 if constexpr (G32) sv[k] *= kSFactor<BITS>;
             }
             if (rl >= uint32_t(ROWS)) continue;
@@ -626,7 +629,7 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
 #pragma unroll
                         for (int k = 0; k < KG; ++k) {
                             if constexpr (G32) op[rt & 1][k] = bf16_codes<BITS>(w[rt & 1][k]);
-                            else op[rt & 1][k] = __builtin_bit_cast(u4, wide_unpack<BITS, CENTRED>(w[rt & 1][k]));
+                            else op[rt & 1][k] = f16_codes<BITS>(w[rt & 1][k], consts);
                         }
                     };
                     f4 d[2][NCT];
@@ -766,9 +769,9 @@ __global__ __launch_bounds__(256) void wide_sum_kernel(const float *__restrict__
     }
 }
 
-template <int BITS, int META, bool G32, bool CENTRED, int NRT, int NCT, int NW>
+template <int BITS, int META, bool G32, int NRT, int NCT, int NW>
 hipError_t launch_instance(const WideParams &p, hipStream_t stream) {
-    auto kernel = wide_mfma_kernel<BITS, META, G32, CENTRED, NRT, NCT, NW>;
+    auto kernel = wide_mfma_kernel<BITS, META, G32, NRT, NCT, NW>;
     constexpr size_t lds = wide_lds_bytes(NRT, NCT, NW);
     const hipError_t e = raise_lds_limit(reinterpret_cast<const void *>(kernel), lds);
     if (e != hipSuccess) return e;
@@ -777,20 +780,12 @@ hipError_t launch_instance(const WideParams &p, hipStream_t stream) {
     return hipGetLastError();
 }
 
-// Centring costs 5% with two RHS tiles, where unpacking no longer hides under
-// the matrix cores (17408x5120, Q4, 128 RHS: 80.7 us, 76.7 without). Q4 does
-// without it there in group 64 with whole 256-column rows; the other shapes'
-// error was lower before (1.8e-7) and they are centred. F16 metadata comes in
-// blocks of up to four RHS only, in group 32.
+// F16 metadata comes in blocks of up to four RHS only, in group 32.
 template <int BITS, int META, bool G32>
 hipError_t launch_tile(const WideParams &p, const WidePlan &pl, hipStream_t stream) {
-#define QMR_WIDE(RT, CT, NW)                                                                                       \
-    if (pl.rt == RT && pl.ct == CT && pl.nw == NW) {                                                               \
-        if constexpr (G32 && (META != 2 || CT == 1)) return launch_instance<BITS, META, G32, true, RT, CT, NW>(p, stream); \
-        if constexpr (!G32 && BITS == 4 && CT == 2)                                                                \
-            if (p.group == 64 && p.cols % 256 == 0) return launch_instance<BITS, META, G32, false, RT, CT, NW>(p, stream); \
-        if constexpr (!G32) return launch_instance<BITS, META, G32, true, RT, CT, NW>(p, stream);                  \
-    }
+#define QMR_WIDE(RT, CT, NW)                                                                                  \
+    if constexpr (META != 2 || CT == 1)                                                                       \
+        if (pl.rt == RT && pl.ct == CT && pl.nw == NW) return launch_instance<BITS, META, G32, RT, CT, NW>(p, stream);
     QMR_WIDE(2, 1, 8) QMR_WIDE(4, 1, 4) QMR_WIDE(4, 1, 8) QMR_WIDE(5, 1, 8) QMR_WIDE(8, 1, 8) QMR_WIDE(8, 1, 4)
     QMR_WIDE(4, 2, 4) QMR_WIDE(4, 2, 8) QMR_WIDE(5, 2, 8) QMR_WIDE(7, 2, 4) QMR_WIDE(8, 2, 4)
 #undef QMR_WIDE

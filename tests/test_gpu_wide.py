@@ -190,3 +190,29 @@ def test_large_columns_do_not_cost_the_others_bits(gpu, rows, cols, bits, group,
     gpu.dispatch("matmul_affine_wide" + NAME[meta], buffers, [rows, cols, bits, group, batch])
     assert gpu.last_hip_kernel() == "wide_mfma_kernel"
     assert (np.abs(gpu.read_f32(buffers[4], batch * rows).reshape(batch, rows) - want) <= bound).all()
+
+
+@pytest.mark.parametrize("bits,group", [(4, 64), (4, 128), (8, 64)])
+def test_columns_of_zeros_change_no_bit(gpu, bits, group):
+    """The arithmetic does not depend on whether the rows are whole 256
+    columns: a matrix and the same one with a group of zeros at its end give
+    the same bits under the same plan."""
+    rows, cols, batch = 70, 512, 40
+    rng = np.random.default_rng(bits * group)
+    w = rng.integers(0, 2**32, (rows, cols * bits // 32), dtype=np.uint32)
+    s = rng.uniform(0.002, 0.02, (rows, cols // group)).astype(np.float32)
+    b = (-(2.0 ** (bits - 1)) * s + rng.normal(0, 1e-3, s.shape)).astype(np.float32)
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    got = []
+    gpu.set_gemv_plan(-6, 401208)
+    try:
+        for extra in (0, group):
+            pad = lambda a, n: np.pad(a, ((0, 0), (0, n))).ravel()
+            buffers = [*upload_matrix(gpu, pad(w, extra * bits // 32), pad(s, extra // group), pad(b, extra // group)),
+                       gpu.upload_f32(pad(x, extra)), gpu.alloc_f32(batch * rows)]
+            gpu.dispatch("matmul_affine_wide", buffers, [rows, cols + extra, bits, group, batch])
+            assert gpu.last_hip_kernel().startswith("wide_mfma_kernel")
+            got.append(gpu.read_f32(buffers[4], batch * rows))
+    finally:
+        gpu.set_gemv_plan(0, 0)
+    assert np.array_equal(got[0], got[1])
