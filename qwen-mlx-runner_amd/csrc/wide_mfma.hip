@@ -129,11 +129,13 @@ constexpr uint32_t img_sums(bool g32) { return 4 * parts_of(g32) * kFragBytes; }
 constexpr uint32_t img_bytes(bool g32) { return img_sums(g32) + 256; }
 constexpr uint32_t kImgFactors = img_sums(false) + 128;
 
-// A wave's piece of LDS: codes on their way to operand order (64 bytes of each
-// row, one unit of Q4 or half a unit of Q8; rows 80 bytes apart so that
-// neither the writes nor the reads meet in a bank).
-constexpr int kCodePitch = 80;
+// A wave's piece of LDS: codes on their way to operand order, 64 bytes of each
+// row (one unit of Q4 or half a unit of Q8). The 16-byte pieces of a row change
+// places with every fourth row, so that neither the writes nor the reads of 16
+// rows meet in a bank.
+constexpr uint32_t kCodePitch = 64;
 constexpr size_t code_bytes(int nrt) { return size_t(16) * nrt * kCodePitch; }
+__device__ __forceinline__ uint32_t code_piece(uint32_t row16, uint32_t piece) { return (piece ^ (row16 >> 2 & 3)) * 16; }
 // A chunk's metadata, two buffers: per row and class four scales, then the
 // same for the biases. The pitch puts the 16 rows of a read in 16 banks (and
 // with four waves and 8 row tiles it leaves room for two workgroups per CU).
@@ -415,7 +417,7 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
     auto put_codes = [&](const u4 (&src)[NRT]) {
 #pragma unroll
         for (int rt = 0; rt < NRT; ++rt)
-            *reinterpret_cast<u4 *>(turn + (rt * 16 + row16) * kCodePitch + piece * 16) = src[rt];
+            *reinterpret_cast<u4 *>(turn + (rt * 16 + row16) * kCodePitch + code_piece(row16, piece)) = src[rt];
     };
     // ---- metadata of chunk c (units u0 + UPC*NW*c ..): item (row, j) = eight
     // consecutive groups of one row, shifted into place when they are used.
@@ -587,8 +589,9 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
     // Codes of K step k of the segment in the turn buffer, row tile rt, as a B operand.
     auto operand = [&](int rt, int k) {
         const unsigned char *row = turn + (rt * 16 + r16) * kCodePitch;
-        if constexpr (BITS == 4) return u2{*reinterpret_cast<const uint32_t *>(row + 16 * k + 4 * q), 0u};
-        else return *reinterpret_cast<const u2 *>(row + 32 * k + 8 * q);
+        const uint32_t r = uint32_t(r16), c = uint32_t(q), s = uint32_t(k);
+        if constexpr (BITS == 4) return u2{*reinterpret_cast<const uint32_t *>(row + code_piece(r, s) + 4 * c), 0u};
+        else return *reinterpret_cast<const u2 *>(row + code_piece(r, 2 * s + (c >> 1)) + 8 * (c & 1));
     };
     // The wave's units of the split, the last one perhaps past it (its loads
     // read zeros): the loop body has no branch, so every wait counts on the
@@ -787,7 +790,7 @@ hipError_t launch_tile(const WideParams &p, const WidePlan &pl, hipStream_t stre
     if constexpr (META != 2 || CT == 1)                                                                       \
         if (pl.rt == RT && pl.ct == CT && pl.nw == NW) return launch_instance<BITS, META, G32, RT, CT, NW>(p, stream);
     QMR_WIDE(2, 1, 8) QMR_WIDE(4, 1, 4) QMR_WIDE(4, 1, 8) QMR_WIDE(5, 1, 8) QMR_WIDE(8, 1, 8) QMR_WIDE(8, 1, 4)
-    QMR_WIDE(4, 2, 4) QMR_WIDE(4, 2, 8) QMR_WIDE(5, 2, 8) QMR_WIDE(7, 2, 4) QMR_WIDE(8, 2, 4)
+    QMR_WIDE(4, 2, 4) QMR_WIDE(4, 2, 8) QMR_WIDE(5, 2, 8) QMR_WIDE(7, 2, 4) QMR_WIDE(8, 2, 4) QMR_WIDE(6, 2, 4) QMR_WIDE(6, 2, 8)
 #undef QMR_WIDE
     return hipErrorNotSupported;
 }
@@ -838,29 +841,34 @@ struct Instance {
     uint32_t rt, ct, nw, per_cu;  // per_cu: workgroups that fit a CU (LDS, registers)
 };
 constexpr Instance kInstances[] = {{2, 1, 8, 1}, {4, 1, 4, 3}, {4, 1, 8, 1}, {5, 1, 8, 1}, {8, 1, 8, 1}, {8, 1, 4, 2},
-                                   {4, 2, 4, 2}, {4, 2, 8, 1}, {5, 2, 8, 1}, {7, 2, 4, 2}, {8, 2, 4, 2}};
+                                   {4, 2, 4, 2}, {4, 2, 8, 1}, {5, 2, 8, 1}, {7, 2, 4, 2}, {8, 2, 4, 2},
+                                   {6, 2, 4, 2}, {6, 2, 8, 1}};
 }  // namespace
 
 // The plan is the cheapest of the compiled instances and up to eight K splits
-// under a model of what a workgroup does, fitted to 1500 timings (17 shapes
-// from 1024x1024 to 17408x5120, 4 to 256 RHS, both code sizes, groups 32, 64
-// and 128; its choice is on average 2.6% slower than the fastest plan, and
-// what is furthest off, 1.4x, are 200 RHS over 900 rows).
+// under a model of what a workgroup does, fitted to the times of every plan of
+// 305 products (14 shapes from 1500x2048 and 512x8192 to 24576x2560 and
+// 17408x5120, 5 to 256 RHS, both code sizes, groups 32, 64 and 128): its choice
+// is on average 0.8% slower than the fastest plan, at worst 19% (24576x2560 Q8
+// with 256 RHS: 129 us, 108 the fastest).
 WidePlan plan_wide(const AffineArgs &a, const DeviceLimits &lim, const WidePlan &force) {
-    // Microseconds: a call, a group's products per row tile (one or two RHS
-    // tiles), the rest of a group step, a metadata chunk, the factor of a CU
-    // with less than two waves per SIMD, a round of workgroups, the sum launch
-    // and its planes per million floats.
-    constexpr float kCall = 6.67f, kStep[2] = {0.091f, 0.133f}, kFix = 0.271f, kChunk = 0.252f, kLone = 1.685f,
-                    kRound = 2.9f, kSum = 6.8f, kPlane = 1.6f;
+    // Microseconds: a group step's products per row tile (one or two RHS
+    // tiles), the factors of group 32 and of Q8 on them, a metadata chunk, the
+    // factor of a CU with less than two waves per SIMD, a round of workgroups,
+    // the sum launch and its planes per million floats.
+    constexpr float kStep[2] = {0.0934f, 0.1404f}, kG32[2] = {0.781f, 0.671f}, kQ8 = 1.187f, kChunk = 0.0525f,
+                    kLone = 1.166f, kRound = 3.31f, kSum = 3.86f, kPlane = 1.74f;
     const uint32_t units = (a.cols + kUnit - 1) / kUnit, nct = (a.batch + 15) / 16;
     const uint32_t steps = a.group == 32 ? 4 : 2;  // group steps per unit
-    const uint32_t cus = uint32_t(std::max(lim.num_cus, 1));
+    // A row block's workgroups all run on one XCD.
+    constexpr uint32_t kXcds = 8;
+    const uint32_t cus = std::max(uint32_t(std::max(lim.num_cus, 1)) / kXcds, 1u);
     WidePlan best;
     float best_us = 0.f;
     for (const Instance &in : kInstances) {
         if (a.meta == Meta::F16 && in.ct != 1) continue;
         if ((force.rt && force.rt != in.rt) || (force.ct && force.ct != in.ct) || (force.nw && force.nw != in.nw)) continue;
+        const float step = float(in.rt) * kStep[in.ct - 1] * (a.group == 32 ? kG32[in.ct - 1] : 1.f) * (a.bits == 8 ? kQ8 : 1.f);
         for (const uint32_t ns : {1u, 2u, 3u, 4u, 6u, 8u}) {
             WidePlan pl;
             pl.rt = in.rt;
@@ -872,13 +880,13 @@ WidePlan plan_wide(const AffineArgs &a, const DeviceLimits &lim, const WidePlan 
             // the encode that allocates nothing, so that both take one plan.
             if (!force.ns && ns > 1 && (units / ns < in.nw || regions(a, pl).total > QMR_STATIC_SCRATCH_BYTES)) continue;
             const uint32_t upw = pl.ups / pl.nw;
-            const uint32_t wgs = (a.rows + 16 * in.rt - 1) / (16 * in.rt) * ((nct + in.ct - 1) / in.ct) * pl.ns;
-            const uint32_t k = (wgs + cus - 1) / cus;  // workgroups on the busiest CU
-            const float unit = float(steps * in.rt) * kStep[in.ct - 1] * (a.group == 32 ? 0.62f : 1.f) + kFix;
-            float us = float(k) * float(in.nw) / 4.f *
-                       (float(upw) * unit + float((upw * steps + 3) / 4) * kChunk);
-            if (std::min(k, in.per_cu) * in.nw < 8) us *= kLone;
-            us += kCall + float((k + in.per_cu - 1) / in.per_cu) * kRound;
+            const float work = float(in.nw) / 4.f * (float(upw * steps) * step + float((upw * steps + 3) / 4) * kChunk);
+            auto round = [&](uint32_t k) {  // k workgroups on a CU at once
+                return k == 0 ? 0.f : float(k) * work * (k * in.nw < 8 ? kLone : 1.f) + kRound;
+            };
+            const uint32_t wgs = ((a.rows + 16 * in.rt - 1) / (16 * in.rt) * pl.ns + kXcds - 1) / kXcds * ((nct + in.ct - 1) / in.ct);
+            const uint32_t full = wgs / (cus * in.per_cu), rest = wgs % (cus * in.per_cu);
+            float us = float(full) * round(in.per_cu) + round((rest + cus - 1) / cus);
             if (pl.ns > 1) us += kSum + float(a.batch) * float(a.rows) * float(pl.ns) * kPlane * 1e-6f;
             if (best.rt == 0 || us < best_us) best = pl, best_us = us;
         }
