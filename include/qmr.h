@@ -136,14 +136,18 @@ int qmr_encode(qmr_command *command, const char *name, qmr_buffer *const *buffer
  * kernel's partial sums and counters, the wide block's activation images)
  * comes from a static scratch array of QMR_STATIC_SCRATCH_BYTES that each GPU
  * holds from library load until the process ends; a launch needing more is
- * rejected with QMR_ERR_INVALID before anything is enqueued. Workspace that
+ * rejected with QMR_ERR_INVALID before anything is enqueued. (Of the wide
+ * blocks these are Q4 ones of group 64 and more than eight RHS over whole 256
+ * columns, codes, scales and biases 16-byte aligned; the others run in
+ * passes over fewer RHS, or as blocks of four, that fit the scratch, and do
+ * so in qmr_encode too.) Workspace that
  * must start at zero (split sums tagged with a fixed epoch, arrival counters)
  * is cleared by a fill kernel inside the call when earlier launches may have
  * left it non-zero: the split-K kernel and the row-band kernel's GEMV and
  * block forms (plain or residual) clear every slot and counter they take, so
  * after the first fill the region stays zero from call to call and needs no
- * fill until the wide block, the row-band MLP form or a failed command has
- * used it. All calls on one GPU share its scratch: calls whose launches
+ * fill until a wide block, a group 32 block of three or four RHS on the wide
+ * kernel, the row-band MLP form or a failed command has used it. All calls on one GPU share its scratch: calls whose launches
  * overlap in time (other streams, other device handles on the same GPU)
  * race. */
 #define QMR_STATIC_SCRATCH_BYTES (8u << 20)
@@ -196,8 +200,9 @@ int qmr_supported_bf16_quantization(uint32_t bits, size_t group);
  *     The reference caps blocks at four RHS (src/gpu.rs:1136-1140). Buffers
  *     w, s, b, x, y; params rows, cols, bits, group, batch with
  *     1 <= batch <= 256; x [batch][cols], y [batch][rows] token-major;
- *     threads = rows*32. Five RHS or more run on MFMA in one pass, fewer as
- *     a block; meant for chunked prefill.
+ *     threads = rows*32. Five RHS or more run on MFMA (with codes that are
+ *     not 16-byte aligned in group 32 only), fewer as a block; meant for
+ *     chunked prefill.
  *   "matmul_affine_add" / "_bf16" / "_f16meta"
  *     y = r + W x, the down projection with the decoder's residual add
  *     (src/engine.rs:764-765). Buffers w, s, b, x, r, y; params as the
@@ -260,9 +265,7 @@ int qmr_supported_bf16_quantization(uint32_t bits, size_t group);
  *            ct*100 + rt (waves per workgroup, K splits, tiles of 16 RHS and
  *            of 16 rows per workgroup; zero fields and ks = 0 leave them to
  *            its planner). Wide blocks of more than four RHS run on that
- *            kernel by default; any other rr runs them as blocks of four,
- *            but for Q4, group 64, F32 or BF16 metadata, whole 256 columns
- *            and more than eight RHS.
+ *            kernel by default; any other rr runs them as blocks of four.
  * Shapes a forced kernel does not support fall back to the next one; pairs
  * that are not compiled fall back to the planner. */
 int qmr_set_gemv_plan(qmr_device *device, int rr, int ks);

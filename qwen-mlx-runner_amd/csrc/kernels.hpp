@@ -239,6 +239,7 @@ bool wide_mfma_supported(const AffineArgs &a);
 // Non-zero fields of `force` (tuning hook) are kept.
 WidePlan plan_wide(const AffineArgs &a, const DeviceLimits &lim, const WidePlan &force = WidePlan{});
 size_t wide_mfma_workspace(const AffineArgs &a, const WidePlan &pl);
+size_t wide_mfma_image_bytes(const AffineArgs &a);  // of 32 RHS; a plan without K splits needs these alone
 hipError_t launch_wide_mfma(const AffineArgs &a, const WidePlan &pl, unsigned char *workspace, hipStream_t stream);
 bool wide_instance(const WidePlan &pl);  // rt, ct and nw are a compiled instance's
 // Host-side walk of every code, image and metadata load the wide contraction

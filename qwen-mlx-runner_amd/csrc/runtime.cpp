@@ -769,15 +769,68 @@ hipError_t launch_product(qmr_device *dev, const qmr::AffineArgs &a, unsigned ch
             return launch_split_k(dev, a, pl, fixed);
         }
     }
-    if (f.rr == 0 && wide_block_preferred(a) && qmr::wide_mfma_supported(a)) {
-        const qmr::WidePlan pl = qmr::plan_wide(a, dev->limits);
-        if (!fixed || qmr::wide_mfma_workspace(a, pl) <= QMR_STATIC_SCRATCH_BYTES) return launch_wide(dev, a, pl, fixed);
-    }
+    if (f.rr == 0 && wide_block_preferred(a) && qmr::wide_mfma_supported(a) &&
+        qmr::wide_mfma_image_bytes(a) <= QMR_STATIC_SCRATCH_BYTES)
+        return launch_wide(dev, a, qmr::plan_wide(a, dev->limits), fixed);
     // The vector-ALU kernels have no fused epilogue.
     ensure(a.residual == nullptr, "fused product needs a matrix-core kernel", QMR_ERR_UNSUPPORTED);
     dev->last_hip = "affine_gemv_kernel";
     start_gpu(dev);
     return qmr::launch_affine_gemv(a, f.rr < -1 ? qmr::GemvPlan{} : f, dev->limits, dev->stream);
+}
+
+// RHS t0 .. t0 + n - 1 of a block (as many as there are).
+qmr::AffineArgs rhs_slice(const qmr::AffineArgs &a, uint32_t t0, uint32_t n) {
+    qmr::AffineArgs sub = a;
+    sub.batch = std::min(n, a.batch - t0);
+    sub.x = a.x + size_t(t0) * a.cols;
+    sub.y = a.y + size_t(t0) * a.rows;
+    return sub;
+}
+
+// The blocks that always take one pass, however large their images:
+// qmr_encode_static rejects them where those don't fit its scratch. The other
+// blocks then take several passes over fewer RHS, in both entries.
+bool wide_one_pass(const qmr::AffineArgs &a) {
+    const uintptr_t al = reinterpret_cast<uintptr_t>(a.w) | reinterpret_cast<uintptr_t>(a.s) |
+                         reinterpret_cast<uintptr_t>(a.b);
+    return a.batch > 8 && a.bits == 4 && a.group == 64 && a.cols % 256 == 0 && al % 16 == 0;
+}
+
+// The wide blocks that run on the wide kernel: five RHS or more of a format it
+// takes. Against blocks of four, eight RHS take 21 us instead of 29 at
+// 17408x5120, 7.4 instead of 8.8 at 1024x1024 (Q4). A forced plan is the block
+// kernels' (rr == -6: this one's).
+bool wide_kernel_takes(const qmr_device *dev, const qmr::AffineArgs &a) {
+    const int rr = dev->forced_plan.rr;
+    return a.batch > 4 && (rr == 0 || rr == -6) && qmr::wide_mfma_supported(a) &&
+           (wide_one_pass(a) || qmr::wide_mfma_image_bytes(a) <= QMR_STATIC_SCRATCH_BYTES);
+}
+
+hipError_t launch_wide_block(qmr_device *dev, const qmr::AffineArgs &a, unsigned char *fixed) {
+    qmr::WidePlan force;
+    if (dev->forced_plan.rr == -6) {
+        const uint32_t ks = uint32_t(dev->forced_plan.ks);
+        force.rt = ks % 100;
+        force.ct = ks / 100 % 10;
+        force.ns = ks / 1000 % 100;
+        force.nw = ks / 100000 % 10;
+    }
+    uint32_t n = a.batch;  // RHS of a pass
+    if (!wide_one_pass(a)) {
+        const size_t pair = qmr::wide_mfma_image_bytes(a);  // of 32 RHS
+        const uint32_t fit = uint32_t(QMR_STATIC_SCRATCH_BYTES / pair), pairs = (a.batch + 31) / 32;
+        const uint32_t passes = (pairs + fit - 1) / fit;
+        n = (pairs + passes - 1) / passes * 32;
+    }
+    hipError_t e = hipSuccess;
+    for (uint32_t t0 = 0; t0 < a.batch && e == hipSuccess; t0 += n) {
+        const qmr::AffineArgs sub = rhs_slice(a, t0, n);
+        qmr::WidePlan pl = qmr::plan_wide(sub, dev->limits, force);
+        if (pl.rt == 0) pl = qmr::plan_wide(sub, dev->limits);  // the pair is not compiled
+        e = launch_wide(dev, sub, pl, fixed);
+    }
+    return e;
 }
 
 }  // namespace
@@ -1359,45 +1412,12 @@ static int encode_command(qmr_command *command, const char *cname, qmr_buffer *c
             a.batch = qmr::starts_with(name, "matmul_") ? params[4] : 1;
             a.meta = meta;
             const bool fast_group = a.group == 32 || a.group == 64 || a.group == 128;
-            // Wide blocks of five RHS on run on the wide kernel: against
-            // blocks of four, eight RHS take 20 us instead of 29 at
-            // 17408x5120, 8.0 instead of 8.5 at 1024x1024 (Q4). A forced plan
-            // is the block kernels' (rr == -6: this one's), and a static
-            // encode whose images don't fit its scratch runs as blocks; the
-            // large blocks of the usual format are refused there instead.
-            qmr::WidePlan wpl;
-            if (wide && a.batch > 4 && qmr::wide_mfma_supported(a)) {
-                const qmr::GemvPlan f = dev->forced_plan;
-                const uintptr_t al = reinterpret_cast<uintptr_t>(a.w) | reinterpret_cast<uintptr_t>(a.s) |
-                                     reinterpret_cast<uintptr_t>(a.b);
-                const bool large = a.batch > 8 && a.bits == 4 && a.group == 64 && a.meta != qmr::Meta::F16 &&
-                                   a.cols % 256 == 0 && al % 16 == 0;
-                if (large || f.rr == 0 || f.rr == -6) {
-                    qmr::WidePlan force;
-                    if (f.rr == -6) {
-                        const uint32_t ks = uint32_t(f.ks);
-                        force.rt = ks % 100;
-                        force.ct = ks / 100 % 10;
-                        force.ns = ks / 1000 % 100;
-                        force.nw = ks / 100000 % 10;
-                    }
-                    wpl = qmr::plan_wide(a, dev->limits, force);
-                    if (wpl.rt == 0) wpl = qmr::plan_wide(a, dev->limits);  // the pair is not compiled
-                    if (fixed && !large && qmr::wide_mfma_workspace(a, wpl) > QMR_STATIC_SCRATCH_BYTES) wpl = {};
-                }
-            }
-            if (wpl.rt > 0) {
-                e = launch_wide(dev, a, wpl, fixed);
+            if (wide && wide_kernel_takes(dev, a)) {
+                e = launch_wide_block(dev, a, fixed);
             } else if (wide) {
-                // Up to four RHS and what the wide kernel doesn't take:
-                // successive blocks of up to four RHS.
-                for (uint32_t t0 = 0; t0 < a.batch && e == hipSuccess; t0 += 4) {
-                    qmr::AffineArgs sub = a;
-                    sub.batch = a.batch - t0 < 4 ? a.batch - t0 : 4;
-                    sub.x = a.x + size_t(t0) * a.cols;
-                    sub.y = a.y + size_t(t0) * a.rows;
-                    e = launch_product(dev, sub, fixed);
-                }
+                // Successive blocks of up to four RHS.
+                for (uint32_t t0 = 0; t0 < a.batch && e == hipSuccess; t0 += 4)
+                    e = launch_product(dev, rhs_slice(a, t0, 4), fixed);
             } else if (dev->reference || !fast_group) {
                 dev->last_hip = "affine_generic_kernel";
                 start_gpu(dev);

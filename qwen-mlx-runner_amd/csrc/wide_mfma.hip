@@ -895,6 +895,9 @@ WidePlan plan_wide(const AffineArgs &a, const DeviceLimits &lim, const WidePlan 
 }
 
 size_t wide_mfma_workspace(const AffineArgs &a, const WidePlan &pl) { return regions(a, pl).total; }
+size_t wide_mfma_image_bytes(const AffineArgs &a) {
+    return size_t((a.cols + kUnit - 1) / kUnit) * 2 * img_bytes(a.group == 32);
+}
 
 WideExtent wide_address_extent(const AffineArgs &a, WidePlan pl) {
     WideExtent out{};

@@ -216,3 +216,28 @@ def test_columns_of_zeros_change_no_bit(gpu, bits, group):
     finally:
         gpu.set_gemv_plan(0, 0)
     assert np.array_equal(got[0], got[1])
+
+
+# Images of 32 RHS: 2.3 MB (Q8), 3.4 MB (group 32), 2.3 MB (ragged columns);
+# the scratch has 8 MiB.
+@pytest.mark.parametrize("rows,cols,bits,group,batch", [(33, 17408, 8, 64, 97), (40, 17408, 4, 32, 130),
+                                                        (17, 17472, 4, 64, 256), (17, 8192, 8, 128, 256)])
+def test_static_entry_runs_the_same_passes(gpu, rows, cols, bits, group, batch):
+    """A wide block whose images pass the static scratch takes several passes
+    over fewer RHS in both entries, with the same bits."""
+    rng = np.random.default_rng(rows + cols + batch)
+    w = rng.integers(0, 2**32, rows * cols * bits // 32, dtype=np.uint32)
+    s = rng.uniform(0.002, 0.02, rows * cols // group).astype(np.float32)
+    b = (-(2.0 ** (bits - 1)) * s + rng.normal(0, 1e-3, s.size)).astype(np.float32)
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    want = oracle.matmul_f64(w, s, b, "f32", x, rows, cols, bits, group, batch, THREADS)
+    got = []
+    for static in (False, True):
+        buffers = [*upload_matrix(gpu, w, s, b), gpu.upload_f32(x.ravel()), gpu.upload_f32(np.full(batch * rows, np.nan))]
+        command = gpu.begin()
+        command.encode("matmul_affine_wide", buffers, [rows, cols, bits, group, batch], rows * 32, 64, static_scratch=static)
+        command.finish()
+        assert gpu.last_hip_kernel() == "wide_mfma_kernel"
+        got.append(gpu.read_f32(buffers[4], batch * rows))
+        assert_gate(got[-1], want)
+    assert np.array_equal(got[0], got[1])
