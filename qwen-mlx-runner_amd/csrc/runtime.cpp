@@ -714,15 +714,16 @@ hipError_t launch_wide(qmr_device *dev, const qmr::AffineArgs &a, const qmr::Wid
 }
 
 // Blocks of three and four RHS in group 32, which the other matrix-core
-// kernels don't take, on the wide kernel instead of the vector-ALU one: where
-// the block's x no longer fits a workgroup's LDS (900x13312 Q4, four RHS: 54
-// us against 15), and, for matrices of more than one round of workgroups,
-// where it leaves room for one or two workgroups per CU (9001x4160 Q4, four
-// RHS: 26.6 us against 19.9; 17408x5120: 51 against 26; Q8 68 against 37).
-// Below the lines the vector-ALU kernel wins: 4096x5120 with four RHS 14.0 us
-// against 14.5, 10000x5120 with three 18.0 against 20.0, 9001x4160 Q8 20.1
-// against 23.4, and small matrices have no use for two launches (1024x1024:
-// 3.5 us against 8.3).
+// kernels don't take, on the wide kernel instead of the vector-ALU one, whose
+// time grows with every RHS and jumps where fewer workgroups fit a CU's LDS
+// beside the block's x (from 20480 floats on one does, from about 40000 on x
+// comes from memory again and again). The wide kernel wins from 37000 floats
+// on (512x13312 Q4, three RHS: 41 us against 15, Q8 23 against 15; below it
+// 5120x8192 with four 18.8 against 20.2), and where the rows make more than one
+// round of the vector-ALU kernel's workgroups, between 5120 rows (5120x5120,
+// four RHS: 14.5 against 15.5) and 7168, from 16384 floats of Q4 (7168x4096, four:
+// 19.9 against 14.5; 10000x5120, three: 17.9 against 21.8) and 20480 of Q8
+// (10000x5120, four: 27.1 against 25.7; 9001x4160, four: 19.7 against 23.1).
 bool wide_block_preferred(const qmr::AffineArgs &a) {
     if (a.group != 32 || a.batch < 3) return false;
     const uint64_t x = uint64_t(a.batch) * a.cols;
@@ -799,11 +800,16 @@ bool wide_one_pass(const qmr::AffineArgs &a) {
 
 // The wide blocks that run on the wide kernel: five RHS or more of a format it
 // takes. Against blocks of four, eight RHS take 21 us instead of 29 at
-// 17408x5120, 7.4 instead of 8.8 at 1024x1024 (Q4). A forced plan is the block
-// kernels' (rr == -6: this one's).
+// 17408x5120, 7.4 instead of 8.8 at 1024x1024 (Q4). Two blocks of a small group
+// 32 matrix on the vector ALU take less than its two launches: up to 4 million
+// weights in rows of up to 2 KB of codes (1024x1024 with eight RHS 6.9 us
+// against 8.4, 2048x2048 9.7 against 10.0; past the lines 4096x2560 16.9 against
+// 11.6, Q8 1024x4096 14.3 against 11.8), and with nine RHS no matrix does
+// (10.6 against 8.4). A forced plan is the block kernels' (rr == -6: this one's).
 bool wide_kernel_takes(const qmr_device *dev, const qmr::AffineArgs &a) {
     const int rr = dev->forced_plan.rr;
-    return a.batch > 4 && (rr == 0 || rr == -6) && qmr::wide_mfma_supported(a) &&
+    const bool small = a.group == 32 && a.batch <= 8 && uint64_t(a.rows) * a.cols <= (4u << 20) && a.cols * a.bits <= 16384;
+    return a.batch > 4 && (rr == -6 || (rr == 0 && !small)) && qmr::wide_mfma_supported(a) &&
            (wide_one_pass(a) || qmr::wide_mfma_image_bytes(a) <= QMR_STATIC_SCRATCH_BYTES);
 }
 

@@ -142,7 +142,7 @@ def test_group_32_keeps_every_bit_of_x(gpu, name, rows, cols, bits, batch):
         assert np.array_equal(kind(got[0]), kind(got[1]))
 
 
-@pytest.mark.parametrize("rows,cols,bits,group,meta,batch", [(65, 1056, 4, 32, "f32", 18), (40, 1056, 8, 32, "bf16", 5),
+@pytest.mark.parametrize("rows,cols,bits,group,meta,batch", [(65, 1056, 4, 32, "f32", 18), (40, 2080, 8, 32, "bf16", 5),
                                                              (65, 1088, 4, 64, "bf16", 18), (40, 1152, 8, 128, "f32", 6)])
 @pytest.mark.parametrize("static", [False, True])
 def test_wide_views_at_four_byte_offsets(gpu, rows, cols, bits, group, meta, batch, static):
@@ -241,3 +241,20 @@ def test_static_entry_runs_the_same_passes(gpu, rows, cols, bits, group, batch):
         got.append(gpu.read_f32(buffers[4], batch * rows))
         assert_gate(got[-1], want)
     assert np.array_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("rows,cols,bits,batch,wide", [(64, 1024, 4, 5, False), (65, 1056, 8, 8, False),
+                                                       (65, 1056, 4, 9, True), (1024, 4096, 4, 8, False),
+                                                       (1025, 4096, 4, 8, True), (1000, 4128, 4, 5, True),
+                                                       (2000, 2080, 8, 5, True), (2048, 2048, 8, 6, False)])
+def test_small_group_32_blocks_run_as_blocks(gpu, rows, cols, bits, batch, wide):
+    """On both sides of the lines in size, in columns and in RHS count."""
+    rng = np.random.default_rng(rows + cols)
+    w = rng.integers(0, 2**32, rows * cols * bits // 32, dtype=np.uint32)
+    s = rng.uniform(0.002, 0.02, rows * cols // 32).astype(np.float32)
+    b = (-(2.0 ** (bits - 1)) * s + rng.normal(0, 1e-3, s.size)).astype(np.float32)
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    buffers = [*upload_matrix(gpu, w, s, b), gpu.upload_f32(x.ravel()), gpu.alloc_f32(batch * rows)]
+    gpu.dispatch("matmul_affine_wide", buffers, [rows, cols, bits, 32, batch])
+    assert (gpu.last_hip_kernel() == "wide_mfma_kernel") == wide
+    assert_gate(gpu.read_f32(buffers[4], batch * rows), oracle.matmul_f64(w, s, b, "f32", x, rows, cols, bits, 32, batch, THREADS))
