@@ -118,10 +118,11 @@ def test_config4_wide_block(gpu, batch):
                                                   (64, 512, 1, "bf16")])
 def test_wide_block_tails_and_metadata(gpu, rows, cols, batch, meta):
     """Wide blocks at ragged row and RHS counts, both wide names, against
-    the FP64 oracle. The kernel's K quarters hold 16 groups at cols 4096 and
-    25 at cols 6400, past one metadata chunk (12 groups for F32 metadata, 20
-    for BF16), so those cases stage several chunks per wave; 17000 rows take
-    the 272-row workgroups and a partial last row block."""
+    the FP64 oracle. A metadata chunk is two 128-column units of every wave:
+    up to 16 units, so that 32 units (4096 columns) and 50 (6400) take several
+    chunks under any plan without K splits; no row count is a multiple of a
+    workgroup's rows but 128 rows, and five RHS and fewer run as blocks or in
+    a single RHS tile."""
     rng = np.random.default_rng(rows + batch)
     w = rng.integers(0, 2**32, rows * cols // 8, dtype=np.uint32)
     sf = rng.uniform(0.002, 0.02, rows * cols // 64).astype(np.float32)

@@ -14,17 +14,19 @@ pytestmark = pytest.mark.gpu
 THREADS = min(16, os.cpu_count() or 1)
 NAME = {"bf16": "_bf16", "f32": ""}
 # (row tiles, RHS tiles, waves) of 16, each with the K splits it is run with.
-SHAPES = [(0, 0, 0, 0), (2, 1, 8, 1), (4, 1, 4, 2), (4, 1, 8, 1), (5, 1, 8, 1), (8, 1, 8, 1), (8, 1, 4, 3),
-          (4, 2, 4, 2), (4, 2, 8, 1), (5, 2, 8, 1), (7, 2, 4, 1), (8, 2, 4, 2)]
+SHAPES = [(0, 0, 0, 0), (2, 1, 8, 1), (4, 1, 4, 2), (4, 1, 8, 1), (5, 1, 8, 1), (8, 1, 8, 2), (8, 1, 4, 3),
+          (4, 2, 4, 2), (4, 2, 8, 1), (5, 2, 8, 2), (6, 2, 4, 1), (6, 2, 8, 2), (7, 2, 4, 1), (8, 2, 4, 2)]
 
 
 # One row more than whole tiles; a last unit of 32, 64 or 128 columns; odd group
 # counts (a BF16 row that starts inside a word); one RHS more than a tile or an
-# image; a matrix of fewer groups than a metadata window's.
+# image; a matrix of fewer groups than a metadata window's; enough units for
+# several metadata chunks of eight waves in each of two K splits.
 @pytest.mark.parametrize("rows,cols,bits,group,meta,batch",
                          [(129, 1056, 4, 32, "bf16", 33), (65, 864, 8, 32, "f32", 17), (81, 1088, 4, 64, "bf16", 5),
                           (257, 1024, 4, 64, "f32", 70), (113, 1984, 8, 64, "bf16", 256), (145, 1408, 4, 128, "bf16", 16),
-                          (33, 640, 8, 128, "f32", 34), (17, 64, 4, 64, "bf16", 6), (8, 128, 8, 128, "f32", 18)])
+                          (33, 640, 8, 128, "f32", 34), (17, 64, 4, 64, "bf16", 6), (8, 128, 8, 128, "f32", 18),
+                          (33, 4288, 4, 64, "bf16", 20), (40, 4480, 8, 128, "f32", 40)])
 def test_wide_shapes_and_formats(gpu, rows, cols, bits, group, meta, batch):
     rng = np.random.default_rng(rows * cols + batch)
     top = 2**bits
@@ -38,7 +40,11 @@ def test_wide_shapes_and_formats(gpu, rows, cols, bits, group, meta, batch):
     # + |b|); a group makes at most 2 * group / 32 products, the scaling and
     # the bias, each rounded to 2^-24 of A, and 32 more join classes and splits.
     per = (np.repeat(np.abs(sf), group) * top + np.repeat(np.abs(bf), group)).reshape(rows, cols) * 1.01
-    bound = (2.0**-21 + (cols / group * (group / 16 + 3) + 32) * 2.0**-24) * (np.abs(x).astype(np.float64) @ per.T)
+    roundings = cols / group * (group / 16 + 3) + 32
+    bound = (2.0**-21 + roundings * 2.0**-24) * (np.abs(x).astype(np.float64) @ per.T)
+    # Over an RHS's rows the roundings are independent, so that they add as
+    # their root, here four times over (x without its lo half: 7e-5).
+    typical = 2.0**-21 + 4 * roundings**0.5 * 2.0**-24
     buffers = [*upload_matrix(gpu, w, s, b), gpu.upload_f32(x.ravel()), gpu.alloc_f32(batch * rows)]
     name, params = "matmul_affine_wide" + NAME[meta], [rows, cols, bits, group, batch]
     try:
@@ -50,6 +56,8 @@ def test_wide_shapes_and_formats(gpu, rows, cols, bits, group, meta, batch):
             got = gpu.read_f32(buffers[4], batch * rows)
             excess = np.abs(got.reshape(batch, rows) - want) / bound
             assert excess.max() <= 1, f"shape {rt} {ct} {nw} splits {ns}: {excess.max():.2f} of the bound"
+            rel = np.linalg.norm(got.reshape(batch, rows) - want, axis=1) / np.linalg.norm(want, axis=1)
+            assert rel.max() <= typical, f"shape {rt} {ct} {nw} splits {ns}: RHS {rel.argmax()} off by {rel.max():.1e}"
             command = gpu.begin()
             command.encode(name, buffers, params, rows * 32, 64, static_scratch=True)
             command.finish()
@@ -58,36 +66,35 @@ def test_wide_shapes_and_formats(gpu, rows, cols, bits, group, meta, batch):
         gpu.set_gemv_plan(0, 0)
 
 
-# On both sides of the lines in rows, in columns and in RHS count.
-@pytest.mark.parametrize("rows,cols,bits,batch,wide", [(7001, 4096, 4, 4, True), (6999, 4096, 4, 4, False),
-                                                       (7000, 4064, 4, 4, False), (7000, 5120, 8, 4, True),
-                                                       (7000, 5088, 8, 4, False), (17, 12320, 4, 3, True),
-                                                       (17, 12288, 8, 3, False), (40, 9248, 8, 4, True),
-                                                       (7000, 20480, 4, 2, False)])
-def test_group_32_blocks_on_either_kernel(gpu, rows, cols, bits, batch, wide):
-    """The default route of a group 32 block and the vector-ALU kernel agree to
-    the bounds of both: four FP32 roundings for each column at the very most."""
+# On both sides of the lines in rows, in columns and in RHS count; odd group
+# counts in 16-bit metadata (4128 and 9248 columns).
+@pytest.mark.parametrize("rows,cols,bits,meta,batch,wide", [(7001, 4096, 4, "f32", 4, True), (6999, 4096, 4, "f32", 4, False),
+                                                            (7000, 4064, 4, "bf16", 4, False), (7000, 5120, 8, "f32", 4, True),
+                                                            (7000, 5088, 8, "f16", 4, False), (17, 12320, 4, "f16", 3, True),
+                                                            (17, 12288, 8, "f32", 3, False), (40, 9248, 8, "bf16", 4, True),
+                                                            (7003, 4128, 4, "f16", 4, True), (7000, 20480, 4, "bf16", 2, False)])
+def test_group_32_blocks_on_either_kernel(gpu, rows, cols, bits, meta, batch, wide):
+    """The default route of a group 32 block, against the FP64 oracle and, bit
+    for bit, through qmr_encode_static."""
     rng = np.random.default_rng(rows + cols)
-    top = 2**bits
     w = rng.integers(0, 2**32, rows * cols * bits // 32, dtype=np.uint32)
-    s = rng.uniform(0.002, 0.02, rows * cols // 32).astype(np.float32)
-    b = (-top / 2 * s + rng.normal(0, 1e-3, s.size)).astype(np.float32)
+    store = {"f32": lambda v: v, "bf16": synth.f32_to_bf16_bits, "f16": lambda v: v.astype(np.float16).view(np.uint16)}[meta]
+    sf = rng.uniform(0.002, 0.02, rows * cols // 32).astype(np.float32)
+    s, b = store(sf), store((-(2.0 ** (bits - 1)) * sf + rng.normal(0, 1e-3, sf.size)).astype(np.float32))
     x = rng.standard_normal((batch, cols)).astype(np.float32)
-    buffers = [*upload_matrix(gpu, w, s, b), gpu.upload_f32(x.ravel()), gpu.alloc_f32(batch * rows)]
+    want = oracle.matmul_f64(w, s, b, meta, x, rows, cols, bits, 32, batch, THREADS)
+    name = "matmul_affine" + {"f32": "", "bf16": "_bf16", "f16": "_f16meta"}[meta]
     got = []
-    try:
-        for plan in ((0, 0), (-1, 0)):
-            print(f"plan {plan}", flush=True)
-            gpu.set_gemv_plan(*plan)
-            gpu.dispatch("matmul_affine", buffers, [rows, cols, bits, 32, batch])
-            if plan == (0, 0):
-                assert (gpu.last_hip_kernel() == "wide_mfma_kernel") == wide
-            got.append(gpu.read_f32(buffers[4], batch * rows).reshape(batch, rows).astype(np.float64))
-    finally:
-        gpu.set_gemv_plan(0, 0)
-    per = (np.repeat(s, 32) * top + np.repeat(np.abs(b), 32)).reshape(rows, cols)
-    bound = 4 * cols * 2.0**-24 * (np.abs(x).astype(np.float64) @ per.T.astype(np.float64))
-    assert (np.abs(got[0] - got[1]) <= bound).all()
+    for static in (False, True):
+        buffers = [*upload_matrix(gpu, w, s, b), gpu.upload_f32(x.ravel()), gpu.alloc_f32(batch * rows)]
+        command = gpu.begin()
+        command.encode(name, buffers, [rows, cols, bits, 32, batch], rows * 32, 64, static_scratch=static)
+        command.finish()
+        assert (gpu.last_hip_kernel() == "wide_mfma_kernel") == wide
+        got.append(gpu.read_f32(buffers[4], batch * rows))
+        assert_gate(got[-1], want)
+    assert np.array_equal(got[0], got[1])
+
 
 # A wide block whose columns fill units, quarters and two RHS tiles, blocks of
 # three and four over the lines that send them to the wide kernel, and the

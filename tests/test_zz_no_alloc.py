@@ -171,9 +171,10 @@ def test_static_band_slots_stay_clear_across_a_sequence_of_calls(gpu):
 
 
 def test_static_entry_rejects_workspace_beyond_the_scratch(gpu):
-    """A wide block of 256 RHS over 17408 columns needs 272*8 images of 8448
-    bytes (18.4 MB) against the 8 MiB scratch: rejected, nothing enqueued
-    (the output keeps its contents), while qmr_encode runs it."""
+    """A wide block of 256 RHS over 17408 columns needs 136 * 16 images of 8448
+    bytes, one for every 128 columns and 16 RHS (18.4 MB), against the 8 MiB
+    scratch: rejected, nothing enqueued (the output keeps its contents), while
+    qmr_encode runs it."""
     rng = np.random.default_rng(9)
     rows, cols, batch = 64, 17408, 256
     name, arrays, params, want = _case(rng, "wide", rows, cols, batch)
