@@ -241,7 +241,7 @@ struct WideParams {
 
 // ---- 1. Activation images: a wave per unit and RHS tile, lane (t16, c4) the
 // columns 8*c4.. of the four K steps of RHS t16. ----
-constexpr uint32_t kPrepWaves = 4;
+constexpr uint32_t kPrepWaves = 1;
 
 // Group 32: parts are cut off, not rounded: three times eight bits are all of
 // a value's, and the first does not overflow. Inf and NaN stay out of the
