@@ -783,11 +783,18 @@ hipError_t launch_instance(const WideParams &p, hipStream_t stream) {
     return hipGetLastError();
 }
 
-// F16 metadata comes in blocks of up to four RHS only, in group 32.
+// The instances of a format. F16 metadata comes in blocks of up to four RHS
+// only, in group 32. Those left out need more than the 256 registers of two
+// waves per SIMD: 12288x4096 Q8 with 256 RHS 117 us with 8 x 2 tiles, 85 with
+// 6 x 2; 5120x5120 Q8 group 32 with 24 RHS 29 us with 7 x 2, 22 with 4 x 2.
+constexpr bool has_instance(int bits, int meta, bool g32, uint32_t rt, uint32_t ct) {
+    return !(meta == 2 && ct > 1) && !(ct > 1 && rt >= 8 && (bits == 8 || g32)) && !(ct > 1 && rt >= 7 && bits == 8 && g32);
+}
+
 template <int BITS, int META, bool G32>
 hipError_t launch_tile(const WideParams &p, const WidePlan &pl, hipStream_t stream) {
 #define QMR_WIDE(RT, CT, NW)                                                                                  \
-    if constexpr (META != 2 || CT == 1)                                                                       \
+    if constexpr (has_instance(BITS, META, G32, RT, CT))                                                      \
         if (pl.rt == RT && pl.ct == CT && pl.nw == NW) return launch_instance<BITS, META, G32, RT, CT, NW>(p, stream);
     QMR_WIDE(2, 1, 8) QMR_WIDE(4, 1, 4) QMR_WIDE(4, 1, 8) QMR_WIDE(5, 1, 8) QMR_WIDE(8, 1, 8) QMR_WIDE(8, 1, 4)
     QMR_WIDE(4, 2, 4) QMR_WIDE(4, 2, 8) QMR_WIDE(5, 2, 8) QMR_WIDE(7, 2, 4) QMR_WIDE(8, 2, 4) QMR_WIDE(6, 2, 4) QMR_WIDE(6, 2, 8)
@@ -847,17 +854,20 @@ constexpr Instance kInstances[] = {{2, 1, 8, 1}, {4, 1, 4, 3}, {4, 1, 8, 1}, {5,
 
 // The plan is the cheapest of the compiled instances and up to eight K splits
 // under a model of what a workgroup does, fitted to the times of every plan of
-// 305 products (14 shapes from 1500x2048 and 512x8192 to 24576x2560 and
+// 485 products (20 shapes from 1500x2048 and 512x8192 to 24576x2560 and
 // 17408x5120, 5 to 256 RHS, both code sizes, groups 32, 64 and 128): its choice
-// is on average 0.8% slower than the fastest plan, at worst 19% (24576x2560 Q8
-// with 256 RHS: 129 us, 108 the fastest).
+// is on average 0.8% slower than the fastest plan (1.1% on products that a fit
+// to the other half has not seen), more than 13% in two only, whose images
+// pass an XCD's L2 (2560x8192 group 32 with 200 RHS: 89 us, 65 in two splits).
 WidePlan plan_wide(const AffineArgs &a, const DeviceLimits &lim, const WidePlan &force) {
-    // Microseconds: a group step's products per row tile (one or two RHS
-    // tiles), the factors of group 32 and of Q8 on them, a metadata chunk, the
-    // factor of a CU with less than two waves per SIMD, a round of workgroups,
-    // the sum launch and its planes per million floats.
-    constexpr float kStep[2] = {0.0934f, 0.1404f}, kG32[2] = {0.781f, 0.671f}, kQ8 = 1.187f, kChunk = 0.0525f,
-                    kLone = 1.166f, kRound = 3.31f, kSum = 3.86f, kPlane = 1.74f;
+    // Microseconds, by RHS tiles of a workgroup where there are two: a group
+    // step's products per row tile, the factors of group 32 and of Q8 on them,
+    // the factor of a CU with less than two waves per SIMD; a metadata chunk, a
+    // workgroup, a round of them, the sum launch and its planes per million
+    // floats.
+    constexpr float kStep[2] = {0.089f, 0.1367f}, kG32[2] = {0.860f, 0.929f}, kQ8[2] = {1.223f, 1.047f},
+                    kLone[2] = {1.942f, 1.160f}, kChunk = 0.0572f, kWork = 0.399f, kRound = 6.71f, kSum = 2.34f,
+                    kPlane = 4.74f;
     const uint32_t units = (a.cols + kUnit - 1) / kUnit, nct = (a.batch + 15) / 16;
     const uint32_t steps = a.group == 32 ? 4 : 2;  // group steps per unit
     // A row block's workgroups all run on one XCD.
@@ -866,9 +876,9 @@ WidePlan plan_wide(const AffineArgs &a, const DeviceLimits &lim, const WidePlan 
     WidePlan best;
     float best_us = 0.f;
     for (const Instance &in : kInstances) {
-        if (a.meta == Meta::F16 && in.ct != 1) continue;
+        if (!has_instance(int(a.bits), a.meta == Meta::F16 ? 2 : 0, a.group == 32, in.rt, in.ct)) continue;
         if ((force.rt && force.rt != in.rt) || (force.ct && force.ct != in.ct) || (force.nw && force.nw != in.nw)) continue;
-        const float step = float(in.rt) * kStep[in.ct - 1] * (a.group == 32 ? kG32[in.ct - 1] : 1.f) * (a.bits == 8 ? kQ8 : 1.f);
+        const float step = float(in.rt) * kStep[in.ct - 1] * (a.group == 32 ? kG32[in.ct - 1] : 1.f) * (a.bits == 8 ? kQ8[in.ct - 1] : 1.f);
         for (const uint32_t ns : {1u, 2u, 3u, 4u, 6u, 8u}) {
             WidePlan pl;
             pl.rt = in.rt;
@@ -880,9 +890,9 @@ WidePlan plan_wide(const AffineArgs &a, const DeviceLimits &lim, const WidePlan 
             // the encode that allocates nothing, so that both take one plan.
             if (!force.ns && ns > 1 && (units / ns < in.nw || regions(a, pl).total > QMR_STATIC_SCRATCH_BYTES)) continue;
             const uint32_t upw = pl.ups / pl.nw;
-            const float work = float(in.nw) / 4.f * (float(upw * steps) * step + float((upw * steps + 3) / 4) * kChunk);
+            const float work = float(in.nw) / 4.f * (float(upw * steps) * step + float((upw * steps + 3) / 4) * kChunk) + kWork;
             auto round = [&](uint32_t k) {  // k workgroups on a CU at once
-                return k == 0 ? 0.f : float(k) * work * (k * in.nw < 8 ? kLone : 1.f) + kRound;
+                return k == 0 ? 0.f : float(k) * work * (k * in.nw < 8 ? kLone[in.ct - 1] : 1.f) + kRound;
             };
             const uint32_t wgs = ((a.rows + 16 * in.rt - 1) / (16 * in.rt) * pl.ns + kXcds - 1) / kXcds * ((nct + in.ct - 1) / in.ct);
             const uint32_t full = wgs / (cus * in.per_cu), rest = wgs % (cus * in.per_cu);
