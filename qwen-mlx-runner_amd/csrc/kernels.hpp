@@ -224,10 +224,10 @@ size_t affine_tile_workspace(const TilePlan &pl, const AffineArgs &a);
 hipError_t launch_affine_tile(const AffineArgs &a, const TilePlan &pl, unsigned long long *partial,
                               uint32_t *counters, uint32_t epoch, const TileWait &wait, hipStream_t stream);
 
-// Wide block on MFMA (Q4/Q8, group 32/64/128, any metadata, batch up to 256):
-// a prep launch converts x into images in `workspace` (wide_mfma_workspace
-// bytes), the contraction, and with K splits the sum of their planes. See
-// wide_mfma.hip.
+// Wide block on MFMA (Q4/Q8, group 32/64/128, F32 or BF16 metadata, batch up to
+// 256; F16 metadata in group 32 up to 16 RHS): a prep launch converts x into
+// images in `workspace` (wide_mfma_workspace bytes), the contraction, and with
+// K splits the sum of their planes. See wide_mfma.hip.
 struct WidePlan {
     uint32_t rt = 0;   // 16-row tiles per workgroup; 0 = no plan
     uint32_t ct = 0;   // 16-RHS tiles per workgroup

@@ -6,9 +6,9 @@
 // D runs on v_mfma_f32_16x16x32_f16 with exact centred codes against x split
 // into hi/lo f16 parts, accurate to 2^-22 of the value and 2^-40 of the largest
 // of its RHS and 64 columns, or, in group 32, on v_mfma_f32_16x16x32_bf16 against
-// the three bf16 parts of x, which are all of it; the scales multiply D in FP32 and the bias term is
-// an FP32 matrix product of S and b (v_mfma_f32_16x16x4_f32 over four groups
-// at a time).
+// the three bf16 parts of x, which are all of it; factors and scales multiply D
+// in FP32 and the bias term is an FP32 matrix product of S and b
+// (v_mfma_f32_16x16x4_f32 over four groups at a time).
 //
 // Launches: wide_prep_kernel (x images), wide_mfma_kernel and, where K is
 // split across workgroups, wide_sum_kernel.
@@ -27,12 +27,13 @@
 //
 // What bounds it: up to 16 RHS the codes (17408x5120, Q4, 5 RHS: 21 us with the
 // prep launch, 50 MB; one wave in flight per SIMD and a prep of 5 us keep it
-// from the 11 us of a copy), then the matrix cores, which spend two products on
-// every code (hi, lo), together with the unpacking: 24 RHS 28 us, 64 RHS 48 us,
-// 128 RHS 75 us, 0.61 PFLOP/s of products. Streaming every operand through LDS
-// and staging it by the whole workgroup took 34, 62 and 73 us; blocks of four,
-// which Q8 and the other groups ran as, 165 us for 64 RHS over a Q8 5120x5120
-// (24 now).
+// from the 11 us of a copy), then issue: two products for every code (hi, lo)
+// and beside 8 of them 18 vector instructions of unpacking, 16 of factors and
+// scales and 8 of staging. 24 RHS 28 us, 64 RHS 49 us, 128 RHS 67 us in long
+// runs, 0.68 PFLOP/s of products. A workgroup of 272 rows x 32 RHS with codes in
+// operand order and without the factors and the centring took 35, 61 and 66 us;
+// blocks of four, which Q8 and the other groups ran as, 145 us for 64 RHS over
+// a Q8 5120x5120 (24 now).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -85,7 +86,7 @@ __device__ __forceinline__ u4 f16_codes(const u2 &w, const CodeConsts<BITS> &c) 
 // columns would be lost beside its large ones. Error against 64 bits at 5120
 // columns 1.5e-7 (Q4) and 1.4e-7 (Q8), on the vector ALU 2.5e-7 and 2.0e-7;
 // with one column 1e4 times the others 1.8e-7 and 1.7e-7 (Q4 in two f16 parts
-// 9e-7). The third part costs 10% at 4 RHS and 24-35% from 64 RHS on.
+// 9e-7). The third part costs 5% at 4 RHS, 21% at 64 and 39% at 200 (9001x4160 Q4).
 template <int BITS>
 __device__ __forceinline__ u4 bf16_codes(const u2 &w) {
     auto pair = [](float lo, float hi) {  // exact: at most eight bits each
@@ -282,7 +283,7 @@ __device__ __forceinline__ void put_image32(float (&xv)[4][8], unsigned char *im
 // The other groups: hi and lo f16 halves under a power of two of its own for
 // every RHS and 64 columns, as the block kernels have it for every group: a
 // column loses bits only where another of the same 64 is 2^17 times larger.
-// (One per RHS and K class: 4e-5 off beside one column of 1e8.)
+// (One per RHS and K class asked that of an eighth of the row.)
 template <int BITS>
 __device__ __forceinline__ void put_image64(const float (&xv)[4][8], unsigned char *img, uint32_t lane) {
 #pragma unroll
@@ -659,7 +660,7 @@ __global__ __launch_bounds__(64 * NW_, 2) void wide_mfma_kernel(WideParams p) {
                         __builtin_amdgcn_sched_barrier(0);
                         // All hi products before the lo ones: half the error
                         // of hi and lo in turn (2.4e-7 against 4.4e-7 at 5120
-                        // columns, Q4), a quarter of lo first.
+                        // columns of uncentred Q4), a quarter of lo first.
 #pragma unroll
                         for (int part = 0; part < PARTS; ++part)
 #pragma unroll
@@ -878,7 +879,8 @@ WidePlan plan_wide(const AffineArgs &a, const DeviceLimits &lim, const WidePlan 
     for (const Instance &in : kInstances) {
         if (!has_instance(int(a.bits), a.meta == Meta::F16 ? 2 : 0, a.group == 32, in.rt, in.ct)) continue;
         if ((force.rt && force.rt != in.rt) || (force.ct && force.ct != in.ct) || (force.nw && force.nw != in.nw)) continue;
-        const float step = float(in.rt) * kStep[in.ct - 1] * (a.group == 32 ? kG32[in.ct - 1] : 1.f) * (a.bits == 8 ? kQ8[in.ct - 1] : 1.f);
+        const float step = float(in.rt) * kStep[in.ct - 1] * (a.group == 32 ? kG32[in.ct - 1] : 1.f) *
+                           (a.bits == 8 ? kQ8[in.ct - 1] : 1.f);
         for (const uint32_t ns : {1u, 2u, 3u, 4u, 6u, 8u}) {
             WidePlan pl;
             pl.rt = in.rt;
@@ -894,7 +896,8 @@ WidePlan plan_wide(const AffineArgs &a, const DeviceLimits &lim, const WidePlan 
             auto round = [&](uint32_t k) {  // k workgroups on a CU at once
                 return k == 0 ? 0.f : float(k) * work * (k * in.nw < 8 ? kLone[in.ct - 1] : 1.f) + kRound;
             };
-            const uint32_t wgs = ((a.rows + 16 * in.rt - 1) / (16 * in.rt) * pl.ns + kXcds - 1) / kXcds * ((nct + in.ct - 1) / in.ct);
+            const uint32_t wgs = ((a.rows + 16 * in.rt - 1) / (16 * in.rt) * pl.ns + kXcds - 1) / kXcds *
+                                 ((nct + in.ct - 1) / in.ct);  // of the busiest XCD
             const uint32_t full = wgs / (cus * in.per_cu), rest = wgs % (cus * in.per_cu);
             float us = float(full) * round(in.per_cu) + round((rest + cus - 1) / cus);
             if (pl.ns > 1) us += kSum + float(a.batch) * float(a.rows) * float(pl.ns) * kPlane * 1e-6f;

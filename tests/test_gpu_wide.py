@@ -43,7 +43,7 @@ def test_wide_shapes_and_formats(gpu, rows, cols, bits, group, meta, batch):
     roundings = cols / group * (group / 16 + 3) + 32
     bound = (2.0**-21 + roundings * 2.0**-24) * (np.abs(x).astype(np.float64) @ per.T)
     # Over an RHS's rows the roundings are independent, so that they add as
-    # their root, here four times over (x without its lo half: 7e-5).
+    # their root, here four times over (x without its lo half: 2e-4).
     typical = 2.0**-21 + 4 * roundings**0.5 * 2.0**-24
     buffers = [*upload_matrix(gpu, w, s, b), gpu.upload_f32(x.ravel()), gpu.alloc_f32(batch * rows)]
     name, params = "matmul_affine_wide" + NAME[meta], [rows, cols, bits, group, batch]
