@@ -252,8 +252,8 @@ def test_pack_bf16_exact_patterns_and_supported_formats():
 WIDE_SHAPES = [(2048, 5120, 4, 64, 128), (16 * 17 * 3 + 5, 512, 4, 64, 33), (9, 256, 4, 64, 1), (300, 1088, 4, 64, 200),
                (129, 1056, 4, 32, 17), (65, 864, 8, 32, 256), (33, 1984, 8, 64, 31), (81, 1408, 4, 128, 16),
                (17, 640, 8, 128, 34), (16, 64, 4, 64, 5), (15, 160, 8, 32, 8), (257, 4224, 8, 128, 70)]
-WIDE_PLANS = [(2, 1, 8), (4, 1, 4), (4, 1, 8), (5, 1, 8), (8, 1, 8), (8, 1, 4), (4, 2, 4), (4, 2, 8), (5, 2, 8), (7, 2, 4),
-              (8, 2, 4)]
+WIDE_PLANS = [(2, 1, 8), (4, 1, 4), (4, 1, 8), (5, 1, 8), (8, 1, 8), (8, 1, 4), (4, 2, 4), (4, 2, 8), (5, 2, 8), (6, 2, 4),
+              (6, 2, 8), (7, 2, 4), (8, 2, 4)]
 
 
 @pytest.mark.parametrize("rows,cols,bits,group,batch", WIDE_SHAPES)

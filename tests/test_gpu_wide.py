@@ -178,17 +178,17 @@ def test_wide_views_at_four_byte_offsets(gpu, rows, cols, bits, group, meta, bat
                                                              (40, 1984, 8, 64, "bf16", 33), (33, 1920, 4, 128, "f32", 20),
                                                              (33, 2176, 8, 128, "bf16", 5)])
 def test_large_columns_do_not_cost_the_others_bits(gpu, rows, cols, bits, group, meta, batch):
-    """Every second group's x is 2^40 times larger under weights of zero, and
+    """Every third group's x is 2^40 times larger under weights of zero, and
     every RHS has a size of its own: the other groups keep their precision."""
     rng = np.random.default_rng(rows * cols)
     top = 2**bits
     w = rng.integers(0, 2**32, rows * cols * bits // 32, dtype=np.uint32)
     sf = rng.uniform(0.002, 0.02, (rows, cols // group)).astype(np.float32)
     bf = (-top / 2 * sf + rng.normal(0, 1e-3, sf.shape)).astype(np.float32)
-    sf[:, 1::2] = bf[:, 1::2] = 0
+    sf[:, 1::3] = bf[:, 1::3] = 0
     s, b = (synth.f32_to_bf16_bits(sf), synth.f32_to_bf16_bits(bf)) if meta == "bf16" else (sf, bf)
     x = (rng.standard_normal((batch, cols)) * np.exp2(rng.integers(-12, 13, (batch, 1)))).astype(np.float32)
-    x *= np.where(np.arange(cols) // group % 2, np.float32(2.0**40), np.float32(1))
+    x *= np.where(np.arange(cols) // group % 3 == 1, np.float32(2.0**40), np.float32(1))
     want = oracle.matmul_f64(w, s.ravel(), b.ravel(), meta, x, rows, cols, bits, group, batch, THREADS).reshape(batch, rows)
     # As in test_wide_shapes_and_formats.
     per = np.repeat(np.abs(sf) * top + np.abs(bf), group, axis=1) * 1.01
